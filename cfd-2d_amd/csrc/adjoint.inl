@@ -414,12 +414,15 @@ __device__ __forceinline__ void rim_d1(D1& RI, D1& EI, D1& PI, D1& UI, D1& VI, D
 
 // Reverse mode of rim (physics.hpp): the VJP of the Riemann solver's five
 // outputs with respect to its eight inputs, for the same evaluated map that
-// rim_d1 differentiates forward -- its values, branches, Newton iterations
-// and shared divisions, each operation reversed.  The iterates are not
+// rim_d1 differentiates forward -- its branches, Newton iterations and shared
+// reciprocals, each operation reversed.  rim_tape evaluates the solver and
+// keeps what the reverse reads (so the primal is evaluated once, not by rim
+// and again here), rim_reverse runs it backwards.  The iterates are not
 // stored: the reverse of Newton iteration k runs the loop again from its
 // start to k (n iterations cost n(n+1)/2 forward iterations).  With more than
-// RIM_REV_MAX iterations it returns false and leaves the work to the caller's
-// forward-mode path.
+// RIM_REV_MAX iterations rim_tape returns false and leaves the work to the
+// caller's forward-mode path.  Divisions are products with the reciprocals
+// that the evaluation formed.
 constexpr int RIM_REV_MAX = 8;
 
 struct RimSetup {
@@ -432,15 +435,15 @@ __device__ __forceinline__ RimSetup rim_setup(double RB, double PB, double UB, d
 	RimSetup f;
 	f.rpB = RB * PB;
 	f.rpE = RE * PE;
-	f.i4 = 1.0 / (f.rpB * f.rpE);
+	f.i4 = rcp_dev(f.rpB * f.rpE);
 	f.iB = f.rpE * f.i4;
 	f.iE = f.rpB * f.i4;
 	f.IRB = PB * f.iB;
 	f.IPB = RB * f.iB;
 	f.IRE = PE * f.iE;
 	f.IPE = RE * f.iE;
-	f.CB = sqrt(K.GAM * PB * f.IRB);
-	f.CE = sqrt(K.GAM * PE * f.IRE);
+	f.CB = sqrt_dev(K.GAM * PB * f.IRB);
+	f.CE = sqrt_dev(K.GAM * PE * f.IRE);
 	f.RCB = RB * f.CB;
 	f.RCE = RE * f.CE;
 	f.EB = f.CB * f.CB * K.ISGAM;
@@ -451,7 +454,7 @@ __device__ __forceinline__ RimSetup rim_setup(double RB, double PB, double UB, d
 
 // one Newton iteration of rim at P: the clamp, both sides' terms, the update
 struct RimNewton {
-	double Pc, x[2], t[2], y[2], den[2], ir, F[2], FS[2], res, S;
+	double Pc, x[2], t[2], y[2], den[2], ir, F[2], FS[2], res, iS;
 	bool clamped, rare[2];
 };
 
@@ -468,7 +471,7 @@ __device__ __forceinline__ RimNewton rim_newton(const RimSetup& f, double P, dou
 		s.y[sd] = side_root(s.t[sd], s.rare[sd], K);
 		s.den[sd] = s.rare[sd] ? K.GAM * s.Pc : RC * s.y[sd] * s.t[sd];
 	}
-	s.ir = 1.0 / (s.den[0] * s.den[1]);
+	s.ir = rcp_dev(s.den[0] * s.den[1]);
 	for (int sd = 0; sd < 2; sd++) {
 		double PK = sd ? PE : PB, C = sd ? f.CE : f.CB;
 		double r = s.den[1 - sd] * s.ir;
@@ -476,7 +479,7 @@ __device__ __forceinline__ RimNewton rim_newton(const RimSetup& f, double P, dou
 		s.FS[sd] = s.rare[sd] ? C * s.y[sd] * r : (K.QGAM * s.x[sd] + K.FGAM) * r * K.IRGAM;
 	}
 	s.res = f.DU - s.F[0] - s.F[1];
-	s.S = s.FS[0] + s.FS[1];
+	s.iS = rcp_dev(s.FS[0] + s.FS[1]);
 	return s;
 }
 
@@ -491,8 +494,8 @@ __device__ __forceinline__ double rim_newton_rev(const RimSetup& f, const RimNew
                                                  const RimConst& K, double Pnb, RimAdj& a)
 {
 	double Pcb = Pnb;
-	double resb = Pnb / s.S;
-	double Sb = -Pnb * s.res / (s.S * s.S);
+	double resb = Pnb * s.iS;
+	double Sb = -resb * s.res * s.iS;
 	a.DU += resb;
 	double yb[2], tb[2], xb[2] = {0.0, 0.0}, denb[2] = {0.0, 0.0}, irb = 0.0;
 	for (int sd = 0; sd < 2; sd++) {
@@ -520,11 +523,12 @@ __device__ __forceinline__ double rim_newton_rev(const RimSetup& f, const RimNew
 		denb[1 - sd] += rb * s.ir;
 		irb += rb * s.den[1 - sd];
 	}
-	double q = s.den[0] * s.den[1], qb = -irb / (q * q);
+	double qb = -irb * s.ir * s.ir;
 	denb[0] += qb * s.den[1];
 	denb[1] += qb * s.den[0];
 	for (int sd = 0; sd < 2; sd++) {
-		double RC = sd ? f.RCE : f.RCB, IPK = sd ? f.IPE : f.IPB;
+		double RC = sd ? f.RCE : f.RCB, IPK = sd ? f.IPE : f.IPB, PK = sd ? PE : PB;
+		double r = s.den[1 - sd] * s.ir;
 		if (s.rare[sd]) {
 			Pcb += denb[sd] * K.GAM;
 		} else {
@@ -532,7 +536,9 @@ __device__ __forceinline__ double rim_newton_rev(const RimSetup& f, const RimNew
 			yb[sd] += denb[sd] * RC * s.t[sd];
 			tb[sd] += denb[sd] * RC * s.y[sd];
 		}
-		tb[sd] += yb[sd] * ((s.rare[sd] ? K.OGAM : 0.5) * s.y[sd] / s.t[sd]);
+		// dy/dt = k y / t, 1/t from den's reciprocal: GAM PK / den or RC y / den
+		double it = r * (s.rare[sd] ? K.GAM * PK : RC * s.y[sd]);
+		tb[sd] += yb[sd] * ((s.rare[sd] ? K.OGAM : 0.5) * s.y[sd] * it);
 		xb[sd] += s.rare[sd] ? tb[sd] : tb[sd] * K.PGAM;
 		Pcb += xb[sd] * IPK;
 		(sd ? a.IPE : a.IPB) += xb[sd] * s.Pc;
@@ -540,95 +546,125 @@ __device__ __forceinline__ double rim_newton_rev(const RimSetup& f, const RimNew
 	return s.clamped ? 0.0 : Pcb;
 }
 
-__device__ __forceinline__ bool rim_vjp(double RB, double PB, double UB, double VB, double RE, double PE, double UE,
-                                        double VE, const RimConst& K, int max_iter, double RIb, double EIb, double PIb,
-                                        double UIb, double VIb, double* xb)
+struct RimTape {
+	RimSetup f;
+	bool vac, rr[2];
+	int n, br;
+	double P0, P, idd;                            // acoustic guess, converged P, 1 / (RCB + RCE)
+	double y[2], t[2], Z[2], M[2], Q[2], den[2], is;  // star states and their shared reciprocal
+	double RI, EI, PI, UI, VI;
+};
+
+__device__ __forceinline__ bool rim_tape(double RB, double PB, double UB, double VB, double RE, double PE, double UE,
+                                         double VE, const RimConst& K, int max_iter, RimTape& T)
 {
 	const double eps = 1.0e-5;
-	RimAdj a{};
-	RimSetup f = rim_setup(RB, PB, UB, RE, PE, UE, K);
-	bool vac = f.DU * K.AGAM < -2.0 * (f.CB + f.CE);
-	double P0 = 0.0, P = 0.0;
-	int n = 0;
-	// star states: y, Z, M, Q, den per side, their shared reciprocal, outputs
-	double yy[2] = {0.0, 0.0}, ts[2] = {0.0, 0.0}, Zs[2] = {0.0, 0.0}, Ms[2] = {0.0, 0.0}, Qs[2] = {0.0, 0.0};
-	double dens[2] = {1.0, 1.0}, is = 0.0;
-	bool rr[2] = {false, false};
+	T.f = rim_setup(RB, PB, UB, RE, PE, UE, K);
+	const RimSetup& f = T.f;
+	T.vac = f.DU * K.AGAM < -2.0 * (f.CB + f.CE);
+	T.n = 0;
+	T.P0 = T.P = T.idd = T.is = 0.0;
 	double Rs[2] = {0.0, 0.0}, Es[2] = {0.0, 0.0}, Us[2] = {0.0, 0.0}, head[2], tail[2];
-	if (vac) {
+	for (int sd = 0; sd < 2; sd++) {
+		T.y[sd] = T.t[sd] = T.Z[sd] = T.M[sd] = T.Q[sd] = 0.0;
+		T.den[sd] = 1.0;
+		T.rr[sd] = false;
+	}
+	if (T.vac) {
 		head[0] = UB - f.CB;
 		tail[0] = UB + 2.0 * f.CB / K.AGAM;
 		tail[1] = UE - 2.0 * f.CE / K.AGAM;
 		head[1] = UE + f.CE;
 	} else {
-		P0 = (PB * f.RCE + PE * f.RCB + f.DU * f.RCB * f.RCE) / (f.RCB + f.RCE);
-		P = P0;
+		T.idd = rcp_dev(f.RCB + f.RCE);
+		T.P0 = (PB * f.RCE + PE * f.RCB + f.DU * f.RCB * f.RCE) * T.idd;
+		double P = T.P0;
 		for (;;) {
 			RimNewton s = rim_newton(f, P, PB, PE, K);
-			P = s.Pc + s.res / s.S;
-			++n;
+			P = s.Pc + s.res * s.iS;
+			++T.n;
 			if (!(fabs(s.res) > eps)) break;
-			if (max_iter > 0 && n >= max_iter) break;
+			if (max_iter > 0 && T.n >= max_iter) break;
 		}
-		if (n > RIM_REV_MAX) return false;
+		T.P = P;
+		if (T.n > RIM_REV_MAX) return false;
 		for (int sd = 0; sd < 2; sd++) {
-			double PK = sd ? PE : PB, IPK = sd ? f.IPE : f.IPB, IRK = sd ? f.IRE : f.IRB, C = sd ? f.CE : f.CB;
+			double PK = sd ? PE : PB, IPK = sd ? f.IPE : f.IPB, C = sd ? f.CE : f.CB;
 			double RK = sd ? RE : RB, sg = sd ? 1.0 : -1.0;
-			rr[sd] = PK > P;
-			ts[sd] = rr[sd] ? P * IPK : (K.TGAM * P + K.HGAM * PK) * IRK;
-			yy[sd] = side_root(ts[sd], rr[sd], K);
-			Zs[sd] = C * yy[sd];
-			Ms[sd] = (-sg) * (RK * yy[sd]);
-			Qs[sd] = PK - P + Ms[sd] * ((-sg) * yy[sd]);
-			dens[sd] = rr[sd] ? K.AGAM * (Zs[sd] * Zs[sd] * K.ISGAM) : Qs[sd] * Ms[sd];
+			T.rr[sd] = PK > P;
+			T.t[sd] = T.rr[sd] ? P * IPK : K.PGAM * (P * IPK) + K.OGAM;
+			T.y[sd] = side_root(T.t[sd], T.rr[sd], K);
+			T.Z[sd] = C * T.y[sd];
+			T.M[sd] = (-sg) * (RK * T.Z[sd]);
+			T.Q[sd] = PK - P + T.M[sd] * ((-sg) * T.Z[sd]);
+			T.den[sd] = T.rr[sd] ? K.AGAM * (T.Z[sd] * T.Z[sd] * K.ISGAM) : T.Q[sd] * T.M[sd];
 		}
-		is = 1.0 / (dens[0] * dens[1]);
+		T.is = rcp_dev(T.den[0] * T.den[1]);
 		for (int sd = 0; sd < 2; sd++) {
 			double C = sd ? f.CE : f.CB, UK = sd ? UE : UB, sg = sd ? 1.0 : -1.0;
-			double r = dens[1 - sd] * is;
-			if (rr[sd]) {
-				Es[sd] = Zs[sd] * Zs[sd] * K.ISGAM;
-				Us[sd] = UK + (sg * K.DGAM) * (Zs[sd] - C);
+			double r = T.den[1 - sd] * T.is, Z = T.Z[sd];
+			if (T.rr[sd]) {
+				Es[sd] = Z * Z * K.ISGAM;
+				Us[sd] = UK + (sg * K.DGAM) * (Z - C);
 				Rs[sd] = P * r;
 				head[sd] = UK + sg * C;
-				tail[sd] = Us[sd] + sg * Zs[sd];
+				tail[sd] = Us[sd] + sg * Z;
 			} else {
-				double IM = Qs[sd] * r, D = UK + sg * yy[sd];
-				Rs[sd] = Ms[sd] * Ms[sd] * Ms[sd] * r;
-				Us[sd] = D + Qs[sd] * IM;
-				Es[sd] = P * Qs[sd] * IM * IM * K.IAGAM;
+				double IM = T.Q[sd] * r, D = UK + sg * Z, M = T.M[sd];
+				Rs[sd] = M * M * M * r;
+				Us[sd] = D + T.Q[sd] * IM;
+				Es[sd] = P * T.Q[sd] * IM * IM * K.IAGAM;
 				head[sd] = D;
 				tail[sd] = D;
 			}
 		}
 	}
 	// sampling (SBL, SFL = head[0], tail[0]; SEL, SSL = head[1], tail[1])
-	double RI, EI;
-	int br;
 	if (head[1] <= 0.0) {
-		br = 0;
-		RI = RE;
-		EI = f.EE;
+		T.br = 0;
+		T.RI = RE;
+		T.EI = f.EE;
+		T.UI = UE;
+		T.VI = VE;
 	} else if (head[0] >= 0.0) {
-		br = 1;
-		RI = RB;
-		EI = f.EB;
+		T.br = 1;
+		T.RI = RB;
+		T.EI = f.EB;
+		T.UI = UB;
+		T.VI = VB;
 	} else if (tail[1] >= 0.0 && tail[0] <= 0.0) {
-		br = Us[1] >= 0.0 ? 2 : 3;
-		RI = br == 2 ? Rs[0] : Rs[1];
-		EI = br == 2 ? Es[0] : Es[1];
+		bool left = Us[1] >= 0.0;
+		T.br = left ? 2 : 3;
+		T.RI = left ? Rs[0] : Rs[1];
+		T.EI = left ? Es[0] : Es[1];
+		T.UI = left ? Us[0] : Us[1];
+		T.VI = left ? VB : VE;
 	} else {
-		br = tail[0] > 0.0 ? 4 : 5;
-		RI = EI = 0.0;  // the fan's values are formed in its reverse below
+		// UI = (UK +- DGGAM sqrt(EK)) IDGAM1, EI = UI^2 ISGAM, RI = RK (EI/EK)^(1/AGAM)
+		// (left fan: K = B and +; right: K = E and -)
+		bool left = tail[0] > 0.0;
+		T.br = left ? 4 : 5;
+		double UK = left ? UB : UE, EK = left ? f.EB : f.EE, RK = left ? RB : RE, pm = left ? 1.0 : -1.0;
+		T.UI = (UK + pm * (K.DGGAM * sqrt(EK))) * K.IDGAM1;
+		T.VI = left ? VB : VE;
+		T.EI = T.UI * T.UI * K.ISGAM;
+		T.RI = RK * pow_iagam(T.EI / EK, K);
 	}
-	// PI = AGAM EI RI; the fans' RI, EI depend on each other, handled there
-	double RIt = RIb, EIt = EIb;
-	if (br < 4) {
-		RIt += PIb * K.AGAM * EI;
-		EIt += PIb * K.AGAM * RI;
-	}
+	T.PI = K.AGAM * T.EI * T.RI;
+	return true;
+}
+
+__device__ __forceinline__ void rim_reverse(const RimTape& T, double RB, double PB, double RE, double PE,
+                                            const RimConst& K, double RIb, double EIb, double PIb, double UIb,
+                                            double VIb, double* xb)
+{
+	RimAdj a{};
+	const RimSetup& f = T.f;
+	double P = T.P;
+	// PI = AGAM EI RI
+	double RIt = RIb + PIb * K.AGAM * T.EI, EIt = EIb + PIb * K.AGAM * T.RI;
 	double Rsb[2] = {0.0, 0.0}, Esb[2] = {0.0, 0.0}, Usb[2] = {0.0, 0.0};
-	switch (br) {
+	switch (T.br) {
 	case 0:
 		a.RE += RIt;
 		a.EE += EIt;
@@ -654,24 +690,17 @@ __device__ __forceinline__ bool rim_vjp(double RB, double PB, double UB, double 
 		a.VE += VIb;
 		break;
 	default: {
-		// UI = (UK +- DGGAM sqrt(EK)) IDGAM1, EI = UI^2 ISGAM, RI = RK (EI/EK)^(1/AGAM),
-		// PI = AGAM EI RI (left fan: K = B and +; right: K = E and -)
-		bool left = br == 4;
-		double UK = left ? UB : UE, EK = left ? f.EB : f.EE, RK = left ? RB : RE, pm = left ? 1.0 : -1.0;
-		double sq = sqrt(EK);
-		double ui = (UK + pm * (K.DGGAM * sq)) * K.IDGAM1;
-		double ei = ui * ui * K.ISGAM;
-		double w = ei / EK, pw = pow_iagam(w, K);
-		double ri = RK * pw;
-		double rib = RIb + PIb * K.AGAM * ei, eib = EIb + PIb * K.AGAM * ri;
-		double pwb = rib * RK;
-		double RKb = rib * pw;
+		bool left = T.br == 4;
+		double EK = left ? f.EB : f.EE, RK = left ? RB : RE, pm = left ? 1.0 : -1.0;
+		double w = T.EI / EK, pw = pow_iagam(w, K);
+		double pwb = RIt * RK;
+		double RKb = RIt * pw;
 		double wb = pwb * (K.IAGAM * pw / w);
-		eib += wb / EK;
-		double EKb = -wb * ei / (EK * EK);
-		double uib = UIb + eib * 2.0 * ui * K.ISGAM;
+		double eib = EIt + wb / EK;
+		double EKb = -wb * T.EI / (EK * EK);
+		double uib = UIb + eib * 2.0 * T.UI * K.ISGAM;
 		double UKb = uib * K.IDGAM1;
-		EKb += pm * uib * K.IDGAM1 * K.DGGAM / (2.0 * sq);
+		EKb += pm * uib * K.IDGAM1 * K.DGGAM / (2.0 * sqrt(EK));
 		if (left) {
 			a.RB += RKb;
 			a.EB += EKb;
@@ -685,28 +714,28 @@ __device__ __forceinline__ bool rim_vjp(double RB, double PB, double UB, double 
 		}
 	}
 	}
-	if (!vac) {
+	if (!T.vac) {
 		// the star states
 		double Pb = 0.0, isb = 0.0, denb[2] = {0.0, 0.0};
-		double yb[2] = {0.0, 0.0}, Zb[2] = {0.0, 0.0}, Mb[2] = {0.0, 0.0}, Qb[2] = {0.0, 0.0};
+		double Zb[2] = {0.0, 0.0}, Mb[2] = {0.0, 0.0}, Qb[2] = {0.0, 0.0};
 		for (int sd = 0; sd < 2; sd++) {
-			double C = sd ? f.CE : f.CB, sg = sd ? 1.0 : -1.0;
-			double r = dens[1 - sd] * is, rb = 0.0;
-			if (rr[sd]) {
-				Zb[sd] += Esb[sd] * 2.0 * Zs[sd] * K.ISGAM;
+			double sg = sd ? 1.0 : -1.0;
+			double r = T.den[1 - sd] * T.is, rb = 0.0;
+			if (T.rr[sd]) {
+				Zb[sd] += Esb[sd] * 2.0 * T.Z[sd] * K.ISGAM;
 				(sd ? a.UE : a.UB) += Usb[sd];
 				Zb[sd] += Usb[sd] * (sg * K.DGAM);
 				(sd ? a.CE : a.CB) -= Usb[sd] * (sg * K.DGAM);
 				Pb += Rsb[sd] * r;
 				rb += Rsb[sd] * P;
 			} else {
-				double IM = Qs[sd] * r, M = Ms[sd], Q = Qs[sd];
+				double IM = T.Q[sd] * r, M = T.M[sd], Q = T.Q[sd];
 				Mb[sd] += Rsb[sd] * 3.0 * M * M * r;
 				rb += Rsb[sd] * M * M * M;
 				double IMb = Usb[sd] * Q;
 				Qb[sd] += Usb[sd] * IM;
-				(sd ? a.UE : a.UB) += Usb[sd];  // D = UK + sg y
-				yb[sd] += Usb[sd] * sg;
+				(sd ? a.UE : a.UB) += Usb[sd];  // D = UK + sg Z
+				Zb[sd] += Usb[sd] * sg;
 				double e2 = Esb[sd] * K.IAGAM;
 				Pb += e2 * Q * IM * IM;
 				Qb[sd] += e2 * P * IM * IM;
@@ -714,53 +743,47 @@ __device__ __forceinline__ bool rim_vjp(double RB, double PB, double UB, double 
 				Qb[sd] += IMb * r;
 				rb += IMb * Q;
 			}
-			denb[1 - sd] += rb * is;
-			isb += rb * dens[1 - sd];
+			denb[1 - sd] += rb * T.is;
+			isb += rb * T.den[1 - sd];
 		}
-		double q = dens[0] * dens[1], qb = -isb / (q * q);
-		denb[0] += qb * dens[1];
-		denb[1] += qb * dens[0];
+		double qb = -isb * T.is * T.is;
+		denb[0] += qb * T.den[1];
+		denb[1] += qb * T.den[0];
+		double itt = rcp_dev(T.t[0] * T.t[1]);
 		for (int sd = 0; sd < 2; sd++) {
-			double C = sd ? f.CE : f.CB, RK = sd ? RE : RB, IPK = sd ? f.IPE : f.IPB, IRK = sd ? f.IRE : f.IRB;
-			double PK = sd ? PE : PB, sg = sd ? 1.0 : -1.0;
-			if (rr[sd]) {
-				Zb[sd] += denb[sd] * K.AGAM * K.ISGAM * 2.0 * Zs[sd];
+			double C = sd ? f.CE : f.CB, RK = sd ? RE : RB, IPK = sd ? f.IPE : f.IPB;
+			double sg = sd ? 1.0 : -1.0;
+			if (T.rr[sd]) {
+				Zb[sd] += denb[sd] * K.AGAM * K.ISGAM * 2.0 * T.Z[sd];
 			} else {
-				Qb[sd] += denb[sd] * Ms[sd];
-				Mb[sd] += denb[sd] * Qs[sd];
+				Qb[sd] += denb[sd] * T.M[sd];
+				Mb[sd] += denb[sd] * T.Q[sd];
 			}
 			(sd ? a.PE : a.PB) += Qb[sd];
 			Pb -= Qb[sd];
-			Mb[sd] += Qb[sd] * ((-sg) * yy[sd]);
-			yb[sd] += Qb[sd] * Ms[sd] * (-sg);
-			(sd ? a.RE : a.RB) += Mb[sd] * (-sg) * yy[sd];
-			yb[sd] += Mb[sd] * (-sg) * RK;
-			(sd ? a.CE : a.CB) += Zb[sd] * yy[sd];
-			yb[sd] += Zb[sd] * C;
-			double tb = yb[sd] * ((rr[sd] ? K.OGAM : 0.5) * yy[sd] / ts[sd]);
-			if (rr[sd]) {
-				Pb += tb * IPK;
-				(sd ? a.IPE : a.IPB) += tb * P;
-			} else {
-				double u = K.TGAM * P + K.HGAM * PK;
-				Pb += tb * IRK * K.TGAM;
-				(sd ? a.PE : a.PB) += tb * IRK * K.HGAM;
-				(sd ? a.IRE : a.IRB) += tb * u;
-			}
+			Mb[sd] += Qb[sd] * ((-sg) * T.Z[sd]);
+			Zb[sd] += Qb[sd] * T.M[sd] * (-sg);
+			(sd ? a.RE : a.RB) += Mb[sd] * (-sg) * T.Z[sd];
+			Zb[sd] += Mb[sd] * (-sg) * RK;
+			(sd ? a.CE : a.CB) += Zb[sd] * T.y[sd];
+			double yb = Zb[sd] * C;
+			double tb = yb * ((T.rr[sd] ? K.OGAM : 0.5) * T.y[sd] * (T.t[1 - sd] * itt));
+			if (!T.rr[sd]) tb *= K.PGAM;
+			Pb += tb * IPK;
+			(sd ? a.IPE : a.IPB) += tb * P;
 		}
 		// the Newton iterations, last to first, each from its recomputed start
-		for (int k = n - 1; k >= 0; k--) {
-			double Pk = P0;
+		for (int k = T.n - 1; k >= 0; k--) {
+			double Pk = T.P0;
 			for (int m = 0; m < k; m++) {
 				RimNewton s = rim_newton(f, Pk, PB, PE, K);
-				Pk = s.Pc + s.res / s.S;
+				Pk = s.Pc + s.res * s.iS;
 			}
 			RimNewton s = rim_newton(f, Pk, PB, PE, K);
 			Pb = rim_newton_rev(f, s, PB, PE, K, Pb, a);
 		}
 		// the acoustic initial guess
-		double num = PB * f.RCE + PE * f.RCB + f.DU * f.RCB * f.RCE, dd = f.RCB + f.RCE;
-		double numb = Pb / dd, ddb = -Pb * num / (dd * dd);
+		double numb = Pb * T.idd, ddb = -numb * T.P0;
 		a.PB += numb * f.RCE;
 		a.RCE += numb * PB;
 		a.PE += numb * f.RCB;
@@ -780,7 +803,8 @@ __device__ __forceinline__ bool rim_vjp(double RB, double PB, double UB, double 
 	a.CB += a.RCB * RB;
 	a.RE += a.RCE * f.CE;
 	a.CE += a.RCE * RE;
-	double abB = a.CB / (2.0 * f.CB), abE = a.CE / (2.0 * f.CE);
+	double icc = 0.5 * rcp_dev(f.CB * f.CE);
+	double abB = a.CB * (f.CE * icc), abE = a.CE * (f.CB * icc);
 	a.PB += abB * K.GAM * f.IRB;
 	a.IRB += abB * K.GAM * PB;
 	a.PE += abE * K.GAM * f.IRE;
@@ -793,7 +817,7 @@ __device__ __forceinline__ bool rim_vjp(double RB, double PB, double UB, double 
 	double iEb = a.IRE * PE + a.IPE * RE;
 	double rpEb = iBb * f.i4, rpBb = iEb * f.i4;
 	double i4b = iBb * f.rpE + iEb * f.rpB;
-	double q4 = f.rpB * f.rpE, q4b = -i4b / (q4 * q4);
+	double q4b = -i4b * f.i4 * f.i4;
 	rpBb += q4b * f.rpE;
 	rpEb += q4b * f.rpB;
 	a.RB += rpBb * PB;
@@ -808,13 +832,12 @@ __device__ __forceinline__ bool rim_vjp(double RB, double PB, double UB, double 
 	xb[5] = a.PE;
 	xb[6] = a.UE;
 	xb[7] = a.VE;
-	return true;
 }
 
-// The exact Godunov flux's vector-Jacobian product.  The solver's primal
-// outputs first (rim), then the flux assembly and the rotation to the normal
-// frame reversed by hand, then the solver itself by rim_vjp.  When the
-// Newton loop ran too long for rim_vjp, forward mode instead: the solver's
+// The exact Godunov flux's vector-Jacobian product.  The solver's outputs
+// first (rim_tape), then the flux assembly and the rotation to the normal
+// frame reversed by hand, then the solver itself (rim_reverse).  When the
+// Newton loop ran too long for that, forward mode instead: the solver's
 // outputs depend on six inputs (density, pressure and normal velocity of
 // each side; the tangential velocities only pass through, VI is VB or VE),
 // so one dual pass (rim_d1) per one of those six, the first also seeding VB,
@@ -826,9 +849,13 @@ __device__ __forceinline__ void godunov_vjp(const Prim& L, const Prim& R, double
 {
 	double unl = L.u * nx + L.v * ny, unr = R.u * nx + R.v * ny;
 	double utl = L.u * ny - L.v * nx, utr = R.u * ny - R.v * nx;
-	double RI, EI, PI, UN, UT;
-	int hit = 0;
-	rim(RI, EI, PI, UN, UT, L.r, L.p, unl, utl, R.r, R.p, unr, utr, K, max_iter, hit);
+	RimTape T;
+	bool taped = rim_tape(L.r, L.p, unl, utl, R.r, R.p, unr, utr, K, max_iter, T);
+	if (!taped) {
+		int hit = 0;
+		rim(T.RI, T.EI, T.PI, T.UI, T.VI, L.r, L.p, unl, utl, R.r, R.p, unr, utr, K, max_iter, hit);
+	}
+	double RI = T.RI, EI = T.EI, PI = T.PI, UN = T.UI, UT = T.VI;
 	// reverse of UI = UN nx + UT ny, VI = UN ny - UT nx, f0 = RI UN,
 	// f1 = f0 UI + PI nx, f2 = f0 VI + PI ny, f3 = (RI (EI + (UI^2 + VI^2)/2) + PI) UN
 	double ui = UN * nx + UT * ny, vi = UN * ny - UT * nx;
@@ -850,7 +877,9 @@ __device__ __forceinline__ void godunov_vjp(const Prim& L, const Prim& R, double
 	double nxb = fb[1] * PI + uib * UN - vib * UT;
 	double nyb = fb[2] * PI + uib * UT + vib * UN;
 	double xb[8];  // adjoints of (RB, PB, UB, VB, RE, PE, UE, VE)
-	if (!rim_vjp(L.r, L.p, unl, utl, R.r, R.p, unr, utr, K, max_iter, RIb, EIb, PIb, UNb, UTb, xb)) {
+	if (taped) {
+		rim_reverse(T, L.r, L.p, R.r, R.p, K, RIb, EIb, PIb, UNb, UTb, xb);
+	} else {
 		const double in[6] = {L.r, L.p, unl, R.r, R.p, unr};
 		double x6[6], sel = 0.0;
 		for (int j = 0; j < 6; j++) {

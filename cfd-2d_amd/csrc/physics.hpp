@@ -38,6 +38,25 @@ __device__ __forceinline__ double sqrt_dev(double x)
 	return (x == 0.0 || x == INFINITY) ? x : g;
 }
 
+// 1/x for the device passes: the hardware reciprocal (2^-23) refined by two
+// Newton-Raphson steps, the last one rounding to within an ulp of 1/x, and
+// the special operands (zero, infinity, NaN) put right by v_div_fixup: six
+// vector instructions where the compiler's IEEE division takes eleven.  The
+// reciprocal of a number at the ends of the exponent range (1/x subnormal,
+// or x subnormal), which no density, pressure or length here comes near, may
+// lose bits.
+__device__ __forceinline__ double rcp_dev(double x)
+{
+	double r = __builtin_amdgcn_rcp(x);
+	r = fma(r, fma(-x, r, 1.0), r);
+	r = fma(r, fma(-x, r, 1.0), r);
+#ifdef __HIP_DEVICE_COMPILE__
+	return __builtin_amdgcn_div_fixup(r, x, 1.0);
+#else
+	return 1.0 / x;  // a host build divides
+#endif
+}
+
 struct Prim {
 	double r, p, u, v;
 };
