@@ -19,7 +19,7 @@ _up = np.ctypeslib.ndpointer(dtype=np.uint32, flags="C_CONTIGUOUS")
 
 K_GRADIENT, K_EDGE_FLUX, K_UPDATE, K_REMEDIATE, K_TAU, K_PRIM = range(6)
 KERNEL_NAMES = ["gradient", "edge_flux", "update", "remediate", "tau", "prim", "impl_gradient", "impl_edge",
-                "impl_assemble"]
+                "impl_assemble", "stage"]
 
 
 class Params(C.Structure):
@@ -463,10 +463,10 @@ class Context:
                 pinned_array((nc, 4), np.float64), pinned_array((nc,), np.float64))
 
     def fuse_gradient(self, mode=True):
-        """Where the gradients are formed: True/1 in the edge pass by each
-        edge's lanes, 2 or "tiled" in the tiled edge pass (once per cell and
-        tile, staged in LDS), False/0 in their own pass, None/-1 the default
-        (edge pass unless a limiter is on); the same results."""
+        """How a stage is split into kernels: None/-1 (default), 2 or "tiled" one
+        kernel by tiles of cells, True/1 an edge pass that forms the gradients
+        and an update pass, False/0 gradient, edge and update passes; the same
+        results."""
         if mode is None:
             m = -1
         elif mode == "tiled" or (not isinstance(mode, bool) and mode == 2):

@@ -1612,36 +1612,37 @@ void launch_fill(cfd2d_ctx* c, double* x, size_t count)
 	hipLaunchKernelGGL(k_fill, dim3((unsigned)((count + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, c->st, x, count, 0.0);
 }
 
-// nsteps forward steps writing every stage's P and G into the stage slots
-// (P slot 0 = primitives of the current state); U advances in place
+// nsteps forward steps writing every stage's P and G into the stage slots,
+// the final state's primitives into the last P slot; U advances in place.
+// The stage kernel stores its stage's input P and G; otherwise the update
+// pass writes the next stage's P, and the stage's gradient records come from
+// the separate gradient pass (fuse mode 0; no limiter here) or from the
+// update pass.
 template <bool MM>
 void record_steps(cfd2d_ctx* c, AdjWork* A, int nsteps)
 {
 	size_t n4 = 4 * (size_t)c->nc, n8 = 8 * (size_t)c->nc;
 	double *P0 = c->b.P, *Po0 = c->b.Po, *G0 = c->b.G;
 	int S = c->p.rk_stages;
-	const int modes2[2] = {UPD_FIRST, UPD_RK2_LAST}, modes3[3] = {UPD_FIRST, UPD_RK3_MID, UPD_RK3_LAST};
+	bool stage = stage_path(c);
 	c->b.P = A->Pst;
 	c->b.Po = A->Pst;
-	launch_prim<MM>(c);
+	if (!stage) launch_prim<MM>(c);
 	size_t t = 0;
 	for (int s = 0; s < nsteps; s++) {
 		for (int st = 0; st < S; st++, t++) {
 			c->b.P = A->Pst + t * n4;
 			c->b.Po = A->Pst + (t + 1) * n4;
 			c->b.G = A->Gst + t * n8;
-			launch_gradient_edge<MM>(c);
-			// the stage's gradient records: the separate gradient pass (fuse mode
-			// 0; no limiter here) has stored them already, otherwise the update
-			// pass forms and stores them
 			c->ph.store_g = c->fuse_mode != 0;
-			launch_update<MM>(c, S == 3 ? modes3[st] : modes2[st]);
+			launch_stage<MM>(c, st);
 			c->ph.store_g = 0;
 		}
 		c->b.P = A->Pst + t * n4;
 		c->b.Po = c->b.P;
 		hipLaunchKernelGGL((k_remediate<MM>), dim3(1), dim3(BLOCK), 0, c->st, c->b, c->ph);
 	}
+	if (stage) launch_prim<MM>(c);
 	c->b.P = P0;
 	c->b.Po = Po0;
 	c->b.G = G0;
@@ -1827,7 +1828,10 @@ int adjoint_run(cfd2d_ctx* c, int nsteps, int ck, const int* mask, double* J, do
 			                   A->seed_w, K, A->seed_p);
 		}
 	};
-	if ((rc = adj_pass(c, c->adj_fwd, key, forward))) return rc;
+	before_steps(c, nsteps);
+	rc = adj_pass(c, c->adj_fwd, key, forward);
+	c->prim_stale = true;  // recorded, not left in b.P
+	if (rc) return rc;
 	std::vector<double> pk(K > 0 ? K : 1);
 	int lim = 0;
 	if (K > 0) HIPCHK(hipMemcpyAsync(pk.data(), A->seed_p, K * sizeof(double), hipMemcpyDeviceToHost, c->st));
@@ -1901,6 +1905,7 @@ int adjoint_run(cfd2d_ctx* c, int nsteps, int ck, const int* mask, double* J, do
 		a.Ws = Ws;
 	};
 	if ((rc = adj_pass(c, c->adj_rev, key, reverse))) return rc;
+	c->prim_stale = false;  // formed at its end
 	if (dJdU0) HIPCHK(hipMemcpyAsync(dJdU0, finT, bytes, hipMemcpyDeviceToHost, c->st));
 	if (dJdbc && c->nbc > 0) {
 		if (a.nbedges > 0)

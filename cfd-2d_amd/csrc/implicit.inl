@@ -84,12 +84,12 @@ __global__ __launch_bounds__(BLOCK) void k_impl_edge(Bufs b, Phys ph)
 	}
 	double f[4];
 	int hit = 0;
-	if (FLUX == CFD2D_FLUX_LAX) flux_lax(f, L, R, nx, ny, ph.gam_flux);
+	if (FLUX == CFD2D_FLUX_LAX) flux_lax(f, L, R, nx, ny, ph.gam_flux, ph.igm1);
 	else flux_godunov(f, L, R, nx, ny, ph.rk, ph.max_newton, hit);
 	if (hit) atomicAdd(&b.err[0], 1ull);
 	double o[4];
 	for (int q = 0; q < 4; q++) o[q] = pair_swap(f[q]);
-	store_edge_flux(b.F, e, gp, f, o, edge_geo(b, e)[2] * 0.5);
+	store_edge_flux(b.F + 4 * (size_t)e + 2 * gp, gp, f, o, edge_geo(b, e)[2] * 0.5);
 }
 
 struct ImplOut {
@@ -206,6 +206,7 @@ extern "C" int cfd2d_implicit_assemble(cfd2d_ctx* c, int steady, double cfl, dou
 	o.cfl = cfl;
 	o.tau = tau;
 	o.steady = steady;
+	refresh_prim(c);
 	rec_start(c, CFD2D_K_IMPL_GRADIENT);
 	if (c->mm) hipLaunchKernelGGL((k_impl_gradient<true>), dim3(grid_of(nc)), dim3(BLOCK), 0, c->st, c->b, c->ph);
 	else hipLaunchKernelGGL((k_impl_gradient<false>), dim3(grid_of(nc)), dim3(BLOCK), 0, c->st, c->b, c->ph);

@@ -67,10 +67,11 @@ struct Prim {
 __device__ __forceinline__ Prim cons_to_prim(double ro, double ru, double rv, double re, const MatV& m)
 {
 	Prim q;
+	double ir = rcp_dev(ro);  // one reciprocal instead of three divisions
 	q.r = ro;
-	q.u = ru / ro;
-	q.v = rv / ro;
-	double E = re / ro;
+	q.u = ru * ir;
+	q.v = rv * ir;
+	double E = re * ir;
 	double e = E - 0.5 * (q.u * q.u + q.v * q.v);
 	q.p = q.r * e * (m.gam - 1);
 	return q;
@@ -164,11 +165,18 @@ __host__ __device__ inline RimConst rim_const(double GAM)
 	return k;
 }
 
+// The solver's functions come in two forms: G14 for GAM = 1.4 alone
+// (RimConst::gamma14), and the general one.  The general powers' exp and log
+// are never reached at GAM = 1.4, but their six inlined copies and the
+// constants they keep in registers were there: without them the Navier-Stokes
+// stage kernel fits its 128 registers and is 60 % shorter.
+
 // x^(1/AGAM) of the fan density (rim_orig: exp(log(x) * (1/AGAM))); x^(5/2)
 // = x^2 sqrt(x) for GAM = 1.4
+template <bool G14 = false>
 __device__ __forceinline__ double pow_iagam(double x, const RimConst& K)
 {
-	if (K.gamma14 && x >= 0.0) return x * x * sqrt_dev(x);
+	if (G14 || (K.gamma14 && x >= 0.0)) return x * x * sqrt_dev(x);
 	return exp(log(x) * K.IAGAM);
 }
 
@@ -179,28 +187,59 @@ __device__ __forceinline__ double pow_iagam(double x, const RimConst& K)
 // seed t^(1/k) (k = 7 or 2) refined by two Newton steps on y^k = t with
 // refined hardware reciprocals of y^(k-1) (quadratic convergence from the
 // ~1e-7 seed to an ulp or two; one refinement of the reciprocal in the first
-// step, whose error the second removes, two in the second).  Other gammas and t
-// outside [1e-30, 1e30] (negative t included) take exp(log(t) OGAM) and the
-// square root.
+// step, whose error the second removes, two in the second): side_root_14.
+// Other gammas and t outside [1e-30, 1e30] (negative t included) take
+// exp(log(t) OGAM) and the square root; G14 takes out t's exponent instead.
+__device__ __forceinline__ double side_root_14(double t, bool rare)
+{
+	float tf = (float)t;
+	double y = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf(tf) * (rare ? (1.0f / 7.0f) : 0.5f));
+	double ik = rare ? (1.0 / 7.0) : 0.5;
+	double y2 = y * y;
+	double pk = rare ? y2 * y2 * y2 : y;  // y^(k-1)
+	double r = __builtin_amdgcn_rcp(pk);
+	r = r * (2.0 - pk * r);
+	y = y + (t * r - y) * ik;
+	y2 = y * y;
+	pk = rare ? y2 * y2 * y2 : y;
+	r = __builtin_amdgcn_rcp(pk);
+	r = r * (2.0 - pk * r);
+	r = r * (2.0 - pk * r);
+	return y + (t * r - y) * ik;
+}
+
+template <bool G14 = false>
 __device__ __forceinline__ double side_root(double t, bool rare, const RimConst& K)
 {
-	if (K.gamma14 && t > 1e-30 && t < 1e30) {
-		float tf = (float)t;
-		double y = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf(tf) * (rare ? (1.0f / 7.0f) : 0.5f));
-		double ik = rare ? (1.0 / 7.0) : 0.5;
+	if ((G14 || K.gamma14) && t > 1e-30 && t < 1e30) return side_root_14(t, rare);
+	if (!rare) return sqrt_dev(t);
+	if (!G14) return exp(log(t) * K.OGAM);
+	if (t == 0.0 || t == INFINITY) return t;
+	if (!(t > 0.0)) return NAN;
+	int e;
+	double m = frexp(t, &e);  // t = m 2^e = (m 2^(e - 7 q)) (2^q)^7
+	int q = e / 7;
+	return ldexp(side_root_14(ldexp(m, e - 7 * q), true), q);
+}
+
+// side_root for the forward solver: within 1e-2 of one (most faces of a
+// smooth flow) the binomial series to e^3 is within 1e-9 of the root and one
+// Newton step from it within rounding, 22 instructions instead of 40
+template <bool G14>
+__device__ __forceinline__ double side_root_fwd(double t, bool rare, const RimConst& K)
+{
+	double e = t - 1.0;
+	if ((G14 || K.gamma14) && fabs(e) < 1e-2) {
+		double a = rare ? (1.0 / 7.0) : 0.5;
+		double y = fma(a * e, fma(fma(a, 0.5, -0.5) * e, fma(fma(a, 1.0 / 3.0, -2.0 / 3.0), e, 1.0), 1.0), 1.0);
 		double y2 = y * y;
-		double pk = rare ? y2 * y2 * y2 : y;  // y^(k-1)
+		double pk = rare ? y2 * y2 * y2 : y;
 		double r = __builtin_amdgcn_rcp(pk);
-		r = r * (2.0 - pk * r);
-		y = y + (t * r - y) * ik;
-		y2 = y * y;
-		pk = rare ? y2 * y2 * y2 : y;
-		r = __builtin_amdgcn_rcp(pk);
-		r = r * (2.0 - pk * r);
-		r = r * (2.0 - pk * r);
-		return y + (t * r - y) * ik;
+		r = fma(r, fma(-pk, r, 1.0), r);
+		r = fma(r, fma(-pk, r, 1.0), r);
+		return y + (t * r - y) * a;
 	}
-	return rare ? exp(log(t) * K.OGAM) : sqrt_dev(t);
+	return side_root<G14>(t, rare, K);
 }
 
 // one side of the Riemann problem: density, pressure, normal velocity, sound
@@ -221,13 +260,14 @@ struct SideNewton {
 	double x, t, y, den;
 };
 
+template <bool G14>
 __device__ __forceinline__ SideNewton side_newton_a(const RimSide& s, double P, const RimConst& K)
 {
 	SideNewton v;
 	v.x = P * s.IP;
 	v.rare = s.P > P;
 	v.t = v.rare ? v.x : K.PGAM * v.x + K.OGAM;
-	v.y = side_root(v.t, v.rare, K);
+	v.y = side_root_fwd<G14>(v.t, v.rare, K);
 	v.den = v.rare ? K.GAM * P : s.RC * v.y * v.t;
 	return v;
 }
@@ -239,30 +279,59 @@ __device__ __forceinline__ void side_newton_b(const RimSide& s, const SideNewton
 	FS = v.rare ? s.C * v.y * r : (K.QGAM * v.x + K.FGAM) * r * K.IRGAM;
 }
 
+// (1 + e)^a for |e| < 1e-3, a = 1/2 or OGAM: the binomial series to e^4 (the
+// next term is below 1e-16)
+__device__ __forceinline__ double near_one_pow(double e, double a)
+{
+	double c4 = fma(a, 0.25, -0.75), c3 = fma(a, 1.0 / 3.0, -2.0 / 3.0), c2 = fma(a, 0.5, -0.5);
+	double q = fma(c4 * e, 1.0, 1.0);
+	q = fma(c3 * e, q, 1.0);
+	q = fma(c2 * e, q, 1.0);
+	return fma(a * e, q, 1.0);
+}
+
+// The root of one side (side_newton_a's y) at the converged P = P1 + dP from
+// the last iteration's, taken at P1: the argument t has changed by the
+// relative amount e = dP / P1 (rarefaction) or dP PGAM / (PK t) (shock), in
+// smooth flow far below 1e-3, and the root by (1 + e)^a.  den's reciprocal r
+// gives 1/P1 and 1/t.  Otherwise, or when the side's wave has changed kind,
+// the root itself: 10 instead of 50 instructions per side, 42 of the solver's
+// 425 per wave each.
+template <bool G14>
+__device__ __forceinline__ double side_root_next(const RimSide& s, const SideNewton& v, double P, double dP, double r,
+                                                 const RimConst& K)
+{
+	bool rare = s.P > P;
+	double e = dP * r * (v.rare ? K.GAM : K.PGAM * s.IP * s.RC * v.y);
+	if (rare == v.rare && fabs(e) < 1e-3) return v.y * near_one_pow(e, rare ? K.OGAM : 0.5);
+	double x = P * s.IP;
+	return side_root<G14>(rare ? x : K.PGAM * x + K.OGAM, rare, K);
+}
+
 // The star state (Rs, Es, Us) of one side at the converged P and its wave's
 // head and tail speeds (src/global.cpp:310-349); sg = -1 for the left side
 // (B), +1 for the right (E).  Rarefaction: Z = C (P/PK)^OGAM, E = Z^2/SGAM,
 // U = UK + sg DGAM (Z - C), R = P / (AGAM E), head UK + sg C, tail U + sg Z.
 // Shock: w = sqrt((TGAM P + HGAM PK)/RK), D = UK + sg w, M = RK (UK - D),
 // Q = PK - P + M (UK - D), R = M^2/Q, U = D + Q/M, E = P Q / (M^2 AGAM),
-// head = tail = D.  One reciprocal per side, 1/(AGAM E) or 1/(Q M) ("den"),
-// the two sides' from one division (side_star_b takes it).
+// head = tail = D.  TGAM P + HGAM PK = GAM PK (PGAM P/PK + OGAM), so w is C
+// times the Newton function's root and both waves take Z = C y.  One
+// reciprocal per side, 1/(AGAM E) or 1/(Q M) ("den"), the two sides' from one
+// division (side_star_b takes it).
 struct SideStar {
 	bool rare;
-	double y, Z, Er, D, M, Q, den;
+	double Z, Er, D, M, Q, den;
 };
 
-__device__ __forceinline__ SideStar side_star_a(const RimSide& s, double P, double sg, const RimConst& K)
+__device__ __forceinline__ SideStar side_star_a(const RimSide& s, double y, double P, double sg, const RimConst& K)
 {
 	SideStar v;
 	v.rare = s.P > P;
-	double t = v.rare ? P * s.IP : (K.TGAM * P + K.HGAM * s.P) * s.IR;
-	v.y = side_root(t, v.rare, K);
-	v.Z = s.C * v.y;
+	v.Z = s.C * y;
 	v.Er = v.Z * v.Z * K.ISGAM;
-	v.D = s.U + sg * v.y;
-	v.M = -sg * s.R * v.y;
-	v.Q = s.P - P + v.M * (-sg * v.y);
+	v.D = s.U + sg * v.Z;
+	v.M = -sg * s.R * v.Z;
+	v.Q = s.P - P + v.M * (-sg * v.Z);
 	v.den = v.rare ? K.AGAM * v.Er : v.Q * v.M;
 	return v;
 }
@@ -287,6 +356,7 @@ __device__ __forceinline__ void side_star_b(const RimSide& s, const SideStar& v,
 	}
 }
 
+template <bool G14 = false>
 __device__ __forceinline__ void rim(double& RI, double& EI, double& PI, double& UI, double& VI, double RB,
                                     double PB, double UB, double VB, double RE, double PE, double UE, double VE,
                                     const RimConst& K, int max_iter, int& hit, int* iters = nullptr)
@@ -298,7 +368,7 @@ __device__ __forceinline__ void rim(double& RI, double& EI, double& PI, double& 
 	double RF, RS, EF, ES, SBL, SFL, SSL, SEL;
 	// 1/rho and 1/p of both sides from one division
 	const double rpB = RB * PB, rpE = RE * PE;
-	const double i4 = 1.0 / (rpB * rpE);
+	const double i4 = rcp_dev(rpB * rpE);
 	const double iB = rpE * i4, iE = rpB * i4;
 	RimSide B, E;
 	B.R = RB; B.P = PB; B.U = UB; B.IR = PB * iB; B.IP = RB * iB;
@@ -323,17 +393,23 @@ __device__ __forceinline__ void rim(double& RI, double& EI, double& PI, double& 
 		SSL = UE - 2.0 * CE / AGAM;
 		SEL = UE + CE;
 	} else {
-		double P = (PB * E.RC + PE * B.RC + DU * B.RC * E.RC) / (B.RC + E.RC);
+		double P = (PB * E.RC + PE * B.RC + DU * B.RC * E.RC) * rcp_dev(B.RC + E.RC), dP;
+		SideNewton nb, ne;
+		double rb, re;  // 1/den of each side
 		int it = 0;
 		for (;;) {
 			if (P < eps) P = eps;
 			double F1, FS1, F2, FS2;
-			SideNewton nb = side_newton_a(B, P, K), ne = side_newton_a(E, P, K);
-			double ir = 1.0 / (nb.den * ne.den);
-			side_newton_b(B, nb, P, ne.den * ir, K, F1, FS1);
-			side_newton_b(E, ne, P, nb.den * ir, K, F2, FS2);
+			nb = side_newton_a<G14>(B, P, K);
+			ne = side_newton_a<G14>(E, P, K);
+			double ir = rcp_dev(nb.den * ne.den);
+			rb = ne.den * ir;
+			re = nb.den * ir;
+			side_newton_b(B, nb, P, rb, K, F1, FS1);
+			side_newton_b(E, ne, P, re, K, F2, FS2);
 			double res = DU - F1 - F2;
-			P = P + res / (FS1 + FS2);
+			dP = res * rcp_dev(FS1 + FS2);
+			P = P + dP;
 			++it;
 			if (!(fabs(res) > eps)) break;
 			if (max_iter > 0 && it >= max_iter) {
@@ -342,8 +418,9 @@ __device__ __forceinline__ void rim(double& RI, double& EI, double& PI, double& 
 			}
 		}
 		if (iters) *iters = it;
-		SideStar sb = side_star_a(B, P, -1.0, K), se = side_star_a(E, P, 1.0, K);
-		double is = 1.0 / (sb.den * se.den);
+		SideStar sb = side_star_a(B, side_root_next<G14>(B, nb, P, dP, rb, K), P, -1.0, K);
+		SideStar se = side_star_a(E, side_root_next<G14>(E, ne, P, dP, re, K), P, 1.0, K);
+		double is = rcp_dev(sb.den * se.den);
 		side_star_b(B, sb, P, -1.0, se.den * is, K, RF, EF, UF, SBL, SFL);
 		side_star_b(E, se, P, 1.0, sb.den * is, K, RS, ES, US, SEL, SSL);
 	}
@@ -361,17 +438,18 @@ __device__ __forceinline__ void rim(double& RI, double& EI, double& PI, double& 
 		UI = (UB + K.DGGAM * sqrt_dev(EB)) * K.IDGAM1;
 		VI = VB;
 		EI = (UI * UI) * K.ISGAM;
-		RI = RB * pow_iagam(EI / EB, K);
+		RI = RB * pow_iagam<G14>(EI * rcp_dev(EB), K);
 	} else {
 		UI = (UE - K.DGGAM * sqrt_dev(EE)) * K.IDGAM1;
 		VI = VE;
 		EI = (UI * UI) * K.ISGAM;
-		RI = RE * pow_iagam(EI / EE, K);
+		RI = RE * pow_iagam<G14>(EI * rcp_dev(EE), K);
 	}
 	PI = AGAM * EI * RI;
 }
 
 // FVM_TVD::calcFlux, Godunov branch (src/methods/fvm_tvd.cpp:602-622)
+template <bool G14 = false>
 __device__ __forceinline__ void flux_godunov(double* f, const Prim& L, const Prim& R, double nx, double ny,
                                              const RimConst& K, int max_iter, int& hit)
 {
@@ -380,7 +458,7 @@ __device__ __forceinline__ void flux_godunov(double* f, const Prim& L, const Pri
 	double utl = L.u * ny - L.v * nx;
 	double utr = R.u * ny - R.v * nx;
 	double RI, EI, PI, UN, UT;
-	rim(RI, EI, PI, UN, UT, L.r, L.p, unl, utl, R.r, R.p, unr, utr, K, max_iter, hit);
+	rim<G14>(RI, EI, PI, UN, UT, L.r, L.p, unl, utl, R.r, R.p, unr, utr, K, max_iter, hit);
 	double UI = UN * nx + UT * ny;
 	double VI = UN * ny - UT * nx;
 	f[0] = RI * UN;
@@ -390,17 +468,18 @@ __device__ __forceinline__ void flux_godunov(double* f, const Prim& L, const Pri
 }
 
 // FLUX=LAX as FVM_TVD_IMPLICIT::calcFlux defines it (src/methods/fvm_tvd_implicit.cpp:939-960)
-__device__ __forceinline__ void flux_lax(double* f, const Prim& L, const Prim& R, double nx, double ny, double GAM)
+__device__ __forceinline__ void flux_lax(double* f, const Prim& L, const Prim& R, double nx, double ny, double GAM,
+                                         double igm1)
 {
 	double unl = L.u * nx + L.v * ny;
 	double unr = R.u * nx + R.v * ny;
-	double al = fabs(unl) + sqrt_dev(GAM * L.p / L.r);
-	double ar = fabs(unr) + sqrt_dev(GAM * R.p / R.r);
+	double al = fabs(unl) + sqrt_dev(GAM * L.p * rcp_dev(L.r));
+	double ar = fabs(unr) + sqrt_dev(GAM * R.p * rcp_dev(R.r));
 	double alpha = al > ar ? al : ar;
 	double rol = L.r, rul = L.r * L.u, rvl = L.r * L.v;
-	double rel = L.p / (GAM - 1.0) + 0.5 * L.r * (L.u * L.u + L.v * L.v);
+	double rel = L.p * igm1 + 0.5 * L.r * (L.u * L.u + L.v * L.v);
 	double ror = R.r, rur = R.r * R.u, rvr = R.r * R.v;
-	double rer = R.p / (GAM - 1.0) + 0.5 * R.r * (R.u * R.u + R.v * R.v);
+	double rer = R.p * igm1 + 0.5 * R.r * (R.u * R.u + R.v * R.v);
 	double frl = rol * unl;
 	double frr = ror * unr;
 	f[0] = 0.5 * (frr + frl - alpha * (ror - rol));
@@ -521,12 +600,14 @@ __device__ __forceinline__ void split_face(const RoeAvg& a, double nx, double ny
 }
 
 // Extension: HLLC (Toro, Riemann Solvers, 3rd ed., 10.4-10.6), Davis wave speeds
-__device__ __forceinline__ void flux_hllc(double* f, const Prim& L, const Prim& R, double nx, double ny, double GAM)
+__device__ __forceinline__ void flux_hllc(double* f, const Prim& L, const Prim& R, double nx, double ny, double GAM,
+                                          double igm1)
 {
 	double unl = L.u * nx + L.v * ny, unr = R.u * nx + R.v * ny;
-	double cl = sqrt_dev(GAM * L.p / L.r), cr = sqrt_dev(GAM * R.p / R.r);
-	double El = L.p / (GAM - 1.0) + 0.5 * L.r * (L.u * L.u + L.v * L.v);
-	double Er = R.p / (GAM - 1.0) + 0.5 * R.r * (R.u * R.u + R.v * R.v);
+	double irl = rcp_dev(L.r), irr = rcp_dev(R.r);
+	double cl = sqrt_dev(GAM * L.p * irl), cr = sqrt_dev(GAM * R.p * irr);
+	double El = L.p * igm1 + 0.5 * L.r * (L.u * L.u + L.v * L.v);
+	double Er = R.p * igm1 + 0.5 * R.r * (R.u * R.u + R.v * R.v);
 	double sl = fmin(unl - cl, unr - cr);
 	double sr = fmax(unl + cl, unr + cr);
 	if (sl >= 0.0) {
@@ -544,14 +625,15 @@ __device__ __forceinline__ void flux_hllc(double* f, const Prim& L, const Prim& 
 		return;
 	}
 	double ml = L.r * (sl - unl), mr = R.r * (sr - unr);
-	double ss = (R.p - L.p + L.r * unl * (sl - unl) - R.r * unr * (sr - unr)) / (ml - mr);
+	double ss = (R.p - L.p + L.r * unl * (sl - unl) - R.r * unr * (sr - unr)) * rcp_dev(ml - mr);
 	const Prim& K = ss >= 0.0 ? L : R;
 	double sk = ss >= 0.0 ? sl : sr;
 	double unk = ss >= 0.0 ? unl : unr;
 	double Ek = ss >= 0.0 ? El : Er;
-	double k = (ss >= 0.0 ? ml : mr) / (sk - ss);
+	double mk = ss >= 0.0 ? ml : mr, irk = ss >= 0.0 ? irl : irr;
+	double k = mk * rcp_dev(sk - ss);
 	double us0 = k, us1 = k * (K.u + (ss - unk) * nx), us2 = k * (K.v + (ss - unk) * ny);
-	double us3 = k * (Ek / K.r + (ss - unk) * (ss + K.p / (K.r * (sk - unk))));
+	double us3 = k * (Ek * irk + (ss - unk) * (ss + K.p * rcp_dev(mk)));
 	double fk0 = K.r * unk, fk1 = K.r * K.u * unk + K.p * nx, fk2 = K.r * K.v * unk + K.p * ny,
 	       fk3 = (Ek + K.p) * unk;
 	f[0] = fk0 + sk * (us0 - K.r);

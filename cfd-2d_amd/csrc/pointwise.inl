@@ -60,8 +60,8 @@ __global__ __launch_bounds__(BLOCK) void k_pointwise(int kind, int n, const doub
 		const double* r = rows + 10 * (size_t)i;
 		Prim L{r[0], r[1], r[2], r[3]}, R{r[4], r[5], r[6], r[7]};
 		double f[4];
-		if (kind == CFD2D_FLUX_LAX) flux_lax(f, L, R, r[8], r[9], K.GAM);
-		else if (kind == CFD2D_FLUX_HLLC) flux_hllc(f, L, R, r[8], r[9], K.GAM);
+		if (kind == CFD2D_FLUX_LAX) flux_lax(f, L, R, r[8], r[9], K.GAM, K.IAGAM);
+		else if (kind == CFD2D_FLUX_HLLC) flux_hllc(f, L, R, r[8], r[9], K.GAM, K.IAGAM);
 		else if (kind == CFD2D_FLUX_ROE) flux_roe(f, L, R, r[8], r[9], K.GAM);
 		else flux_godunov(f, L, R, r[8], r[9], K, max_newton, hit);
 		double* o = out + 4 * (size_t)i;

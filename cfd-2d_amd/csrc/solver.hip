@@ -15,8 +15,8 @@
 //          the update pass reads only the faces),
 //          lsqw[nc][6] least-squares weights (wx wy per face), cfn[nc][6]
 //          the faces' outward n l (Green-Gauss weights), both one 48 B
-//          record per cell (three 16-byte loads), cgp[12][nc] the cell's offsets
-//          to its faces' Gauss points (limiter only), flags[nc]
+//          record per cell (three 16-byte loads), cmid[4][nc] the cell's offsets
+//          to its first two faces' midpoints (limiter only), flags[nc]
 //   edges  eg[ne][4] one 32 B record per edge: unit normal out of c1 and
 //          length (nx, ny, l), then the two cells c1, c2 as two ints in the
 //          last 8 bytes (c2 = -(bc+1) on a boundary),
@@ -26,12 +26,14 @@
 //          c1 at Gauss point 2, then zeros),
 //          F[ne][4] = (flux at gp1 + flux at gp2) * l/2, one record per edge
 //          written once
-// Each RK stage is three passes: gradient (cell gather), edge flux (a lane
-// pair per edge, result written once to F), update (cell gather of its
-// three faces in ascending edge order, then the RK combination); without a
-// limiter the edge pass forms the two cells' gradients itself and the
-// gradient pass is not run.  No floating-point atomics: results do not
-// depend on scheduling.
+// A RK stage is one launch of k_stage, which works by tiles of neighbouring
+// cells and has arrays of its own for them (Bufs), or, where asked for
+// (cfd2d_fuse_gradient), three passes: gradient (cell gather), edge flux (a
+// lane pair per edge, result written once to F), update (cell gather of its
+// three faces in ascending edge order, then the RK combination); in mode 1
+// the edge pass forms the two cells' gradients itself and the gradient pass is
+// not run.  The same bits either way.  No floating-point atomics: results do
+// not depend on scheduling.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -57,7 +59,7 @@ constexpr int NXCD = 8;
 
 struct Bufs {
 	int nc, ne, nblocks, nmat;
-	double *U, *U0, *P, *Po, *G, *dtS, *S, *lsqw, *cfn, *cgp, *loc, *R;
+	double *U, *U0, *P, *Po, *G, *dtS, *S, *lsqw, *cfn, *cmid, *loc, *R;
 	double* Un;  // where the update pass writes the stage's state (launch_update)
 	int *cface, *cnb, *cmat;
 	unsigned* flags;
@@ -69,14 +71,20 @@ struct Bufs {
 	double* bcpar;
 	double* mtab;  // 5 per material: M, Cv, gam, mu, kc
 	unsigned long long* err;  // [0] Newton cap hits, [1] non-finite cells
-	// tiled edge pass (k_edge_tile): per tile (int4) the first of its staged
-	// cells in tcell, their count, its first edge and edge count; tcell the
-	// staged cells of every tile, ascending; eslot per edge the LDS rows of
-	// c1 (low 16 bits) and c2 (high 16 bits, 0xffff on a boundary)
-	int* tiles;
-	int* tcell;
-	unsigned* eslot;
-	int ntiles;  // 0: the edges are not in c1 order, no tiled pass
+	// stage pass (k_stage): every tile's arrays start at tile * tall (all its
+	// cells), tile * tsc (staged cells) or tile * tec (edges), so addresses
+	// follow from the block index.
+	double* U1;     // second stage buffer (three stages)
+	int4* thead;    // per tile: own cells, staged cells, all cells, edges
+	int* tcell;     // per cell: the cell
+	int4* trec;     // per staged cell: the tile's cell across each face in ascending edge order
+	                // (-1 - edge on a boundary), then the cell
+	double* tw;     // [.][6] its gradient weights (lsqw or cfn, by the context's gradient)
+	double* tcmid;  // [tile][4][tsc] its offsets to its first two faces' midpoints (limiter only)
+	int2* tface;    // per own cell: its faces as (edge of the tile) * 2 + side, 16 bits each
+	double* tgeo;   // [.][4] per edge: nx, ny, length with the sign of edge_offset, edge_pack
+	double* tmid;   // [.][2][2] per edge: its midpoint from the two lanes' cells
+	int ntiles, tall, tsc, tec, tthreads;
 };
 
 struct Phys {
@@ -126,6 +134,12 @@ __device__ __forceinline__ void st4(double* base, size_t i, const double* v)
 	p[1] = v[1];
 	p[2] = v[2];
 	p[3] = v[3];
+}
+
+__device__ __forceinline__ void ld6(const double* rec, double* v)
+{
+	const double* p = static_cast<const double*>(__builtin_assume_aligned(rec, 16));
+	for (int q = 0; q < 6; q++) v[q] = p[q];
 }
 
 __device__ __forceinline__ void ld8(const double* base, size_t i, double* v)
@@ -182,6 +196,30 @@ __device__ __forceinline__ int2 edge_cells(const Bufs& b, size_t e)
 __host__ __device__ __forceinline__ size_t edl_index(size_t e, int side, int g)
 {
 	return side ? 8 * e + 4 + 2 * (1 - g) : 8 * e + 2 * g;
+}
+
+// Gauss points of an edge from its midpoint (mx, my): mid -+ l/(2 sqrt(3))
+// along the edge (MeshReaderSalomeUnv.cpp:158-169), whose direction is the
+// normal turned, (-ny, nx), times the sign sl carries (sl = +-l).  Offset of
+// the first Gauss point, and of the second with the other sign.  Every
+// product and sum is rounded by itself, so the host, which fills edl, and
+// the stage kernel, which forms the offsets from the midpoint, agree bitwise.
+__host__ __device__ __forceinline__ void edge_offset(double mx, double my, double nx, double ny, double sl, int second,
+                                                     double* o)
+{
+#pragma clang fp contract(off)
+	const double k = 0.28867513459481287;  // 1 / (2 sqrt(3))
+	double h = second ? -(sl * k) : sl * k;
+	double dx = h * ny, dy = h * nx;
+	o[0] = mx + dx;
+	o[1] = my - dy;
+}
+
+// an edge of a tile: staged cells of its lanes (second: -1 - boundary object)
+// and whether this tile reports its Newton cap hits
+__host__ __device__ __forceinline__ int2 edge_pack(int s1, int s2, bool report)
+{
+	return make_int2(s1 << 1 | (report ? 1 : 0), s2);
 }
 
 // the cell's faces and neighbours (one 16-byte record each)
@@ -248,12 +286,14 @@ __device__ __forceinline__ void sta8(double* base, size_t n, size_t i, const dou
 	for (int q = 0; q < 8; q++) base[q * n + i] = v[q];
 }
 
-__device__ __forceinline__ Prim load_prim(const Bufs& b, int i)
+__device__ __forceinline__ Prim load_prim_from(const double* P, int i)
 {
 	double v[4];
-	ld4(b.P, i, v);
+	ld4(P, i, v);
 	return Prim{v[0], v[1], v[2], v[3]};
 }
+
+__device__ __forceinline__ Prim load_prim(const Bufs& b, int i) { return load_prim_from(b.P, i); }
 
 __device__ __forceinline__ void store_prim_to(double* P, size_t, int i, const Prim& q)
 {
@@ -263,16 +303,36 @@ __device__ __forceinline__ void store_prim_to(double* P, size_t, int i, const Pr
 
 __device__ __forceinline__ void store_prim(const Bufs& b, int i, const Prim& q) { store_prim_to(b.P, b.nc, i, q); }
 
+// a boundary object's type and parameters
+struct Bound {
+	int type;
+	double par[4];
+};
+
+__device__ __forceinline__ Bound load_bound(const Bufs& b, int bc)
+{
+	Bound o;
+	o.type = b.bctype[bc];
+	ld4(b.bcpar, bc, o.par);
+	return o;
+}
+
+// ghost of a (cell-centre or reconstructed) state at a boundary, normal (nx, ny)
+__device__ __forceinline__ Prim ghost_at(const Bound& o, double nx, double ny, const Prim& inside, const Prim& centre,
+                                         const MatV& m)
+{
+	double Tc = temperature(centre, m);
+	double czc = sqrt(m.gam * centre.p / centre.r);
+	return ghost_state(o.type, o.par, nx, ny, inside, Tc, czc, m);
+}
+
 // ghost of cell i's (cell-centre or reconstructed) state across boundary edge e
 template <bool MM>
 __device__ __forceinline__ Prim ghost_of(const Bufs& b, const Phys& ph, int e, int c1, const Prim& inside,
                                          const Prim& centre)
 {
-	int bc = -edge_cells(b, e).y - 1;
-	MatV m = mat_of<MM>(b, ph, c1);
-	double Tc = temperature(centre, m);
-	double czc = sqrt(m.gam * centre.p / centre.r);
-	return ghost_state(b.bctype[bc], &b.bcpar[4 * bc], edge_geo(b, e)[0], edge_geo(b, e)[1], inside, Tc, czc, m);
+	return ghost_at(load_bound(b, -edge_cells(b, e).y - 1), edge_geo(b, e)[0], edge_geo(b, e)[1], inside, centre,
+	                mat_of<MM>(b, ph, c1));
 }
 
 // ---------------------------------------------------------------- kernels
@@ -297,40 +357,50 @@ __global__ __launch_bounds__(BLOCK) void k_prim(Bufs b, Phys ph)
 }
 
 // Barth-Jespersen scaling with minmod(1, r) at the cell's six Gauss points
-// (extension; the oracle's limit_minmod)
-__device__ __forceinline__ void minmod_limit(const Bufs& b, int i, const int* face, const Prim& pi,
-                                             const Prim* nb, double* g)
+// (extension; the oracle's limit_minmod).  The points' offsets from the
+// centroid follow from those of two face midpoints, m0 and m1 (component
+// arrays, coalesced: component q of cell i at cmid[q n + i]): the three
+// midpoints' sum to nothing, and face k's Gauss points lie at m_k -+
+// (m_i - m_j) / sqrt(3), the other two midpoints' difference being half the
+// face's vector.  32 bytes per cell instead of the six offsets' 96, and 16
+// registers fewer.
+__device__ __forceinline__ void minmod_limit(const double* cmid, size_t n, size_t i, const Prim& pi, const Prim* nb,
+                                             double* g)
 {
-	double phi[4] = {pi.r, pi.p, pi.u, pi.v};
-	double lo[4], hi[4];
-	for (int q = 0; q < 4; q++) lo[q] = hi[q] = phi[q];
-	for (int k = 0; k < 3; k++) {
-		double v[4] = {nb[k].r, nb[k].p, nb[k].u, nb[k].v};
-		for (int q = 0; q < 4; q++) {
-			if (v[q] < lo[q]) lo[q] = v[q];
-			if (v[q] > hi[q]) hi[q] = v[q];
+	const double s = 0.57735026918962573;  // 1 / sqrt(3)
+	double m0x = cmid[i], m0y = cmid[n + i], m1x = cmid[2 * n + i], m1y = cmid[3 * n + i];
+	double up[4], down[4];  // largest minus own, own minus smallest
+	for (int q = 0; q < 4; q++) {
+		double phi = q == 0 ? pi.r : q == 1 ? pi.p : q == 2 ? pi.u : pi.v;
+		double lo = phi, hi = phi;
+		for (int k = 0; k < 3; k++) {
+			double v = q == 0 ? nb[k].r : q == 1 ? nb[k].p : q == 2 ? nb[k].u : nb[k].v;
+			if (v < lo) lo = v;
+			if (v > hi) hi = v;
 		}
-	}
-	double d[6][2];  // offsets to the Gauss points of the faces, per cell (coalesced)
-	size_t n = b.nc;
-	for (int k = 0; k < 6; k++) {
-		d[k][0] = b.cgp[(size_t)(2 * k) * n + i];
-		d[k][1] = b.cgp[(size_t)(2 * k + 1) * n + i];
+		up[q] = hi - phi;
+		down[q] = phi - lo;
 	}
 	// psi = min(1, min_k r_k), r_k = (hi - phi) / D or (lo - phi) / D by the sign
 	// of D, always >= 0: the smallest ratio is picked by cross-multiplied
 	// comparisons (a_k den < num b_k, all terms >= 0) and divided once
 	for (int q = 0; q < 4; q++) {
 		double gx = g[2 * q], gy = g[2 * q + 1];
+		double A[3];  // the gradient along each midpoint's offset
+		A[0] = gx * m0x + gy * m0y;
+		A[1] = gx * m1x + gy * m1y;
+		A[2] = -(A[0] + A[1]);
 		double num = 1.0, den = 1.0;
-		for (int k = 0; k < 6; k++) {
-			double D = gx * d[k][0] + gy * d[k][1];
-			if (D == 0.0) continue;
-			double a = D > 0.0 ? hi[q] - phi[q] : phi[q] - lo[q];
-			double bb = fabs(D);
-			if (a * den < num * bb) {
-				num = a;
-				den = bb;
+		for (int k = 0; k < 3; k++) {
+			double h = s * (A[(k + 1) % 3] - A[(k + 2) % 3]);
+			for (int e = 0; e < 2; e++) {
+				double D = e ? A[k] + h : A[k] - h;
+				double a = D > 0.0 ? up[q] : down[q];
+				double bb = fabs(D);
+				if (D != 0.0 && a * den < num * bb) {
+					num = a;
+					den = bb;
+				}
 			}
 		}
 		double psi = num / den;
@@ -343,23 +413,15 @@ __device__ __forceinline__ void minmod_limit(const Bufs& b, int i, const int* fa
 // Green-Gauss gradients, FVM_TVD::calcGrad (src/methods/fvm_tvd.cpp:242-301)
 // as a gather: the faces of cell i in ascending edge order, each adding
 // (phi_c1 + phi_c2)/2 * n * l with + on c1's side and - on c2's, then / S.
-// LSQ (extension): grad = sum_k w_k (phi_k - phi_i).  pi, face and nb (the
+// LSQ (extension): grad = sum_k w_k (phi_k - phi_i).  pi and nb (the
 // neighbour states, ghosts on a boundary) are returned for the limiter.
-template <bool MM, bool LSQ>
-__device__ __forceinline__ void cell_gradient(const Bufs& b, const Phys& ph, int i, Prim& pi, int* face, Prim* nb,
-                                              double* g)
+//
+// gradient_sum: from the cell's state, its neighbours' and its weight record w
+template <bool LSQ>
+__device__ __forceinline__ void gradient_sum(const double* w, const Prim& pi, const Prim* nb, double S, double* g)
 {
-	pi = load_prim(b, i);
 	for (int q = 0; q < 8; q++) g[q] = 0.0;
-	CellTop tp = load_top(b, i);
-	for (int k = 0; k < 3; k++) {
-		face[k] = tp.f[k];
-		int j = tp.nb[k];
-		if (j >= 0) nb[k] = load_prim(b, j);
-		else nb[k] = ghost_of<MM>(b, ph, face[k] >> 1, i, pi, pi);
-	}
 	if (LSQ) {
-		const double* w = static_cast<const double*>(__builtin_assume_aligned(b.lsqw + 6 * (size_t)i, 16));
 		for (int k = 0; k < 3; k++) {
 			double wx = w[2 * k], wy = w[2 * k + 1];
 			double dphi[4] = {nb[k].r - pi.r, nb[k].p - pi.p, nb[k].u - pi.u, nb[k].v - pi.v};
@@ -369,7 +431,6 @@ __device__ __forceinline__ void cell_gradient(const Bufs& b, const Phys& ph, int
 			}
 		}
 	} else {
-		const double* w = static_cast<const double*>(__builtin_assume_aligned(b.cfn + 6 * (size_t)i, 16));
 		for (int k = 0; k < 3; k++) {
 			// n l out of cell i (the reference adds for c1 and subtracts for c2)
 			double fx = w[2 * k], fy = w[2 * k + 1];
@@ -379,9 +440,24 @@ __device__ __forceinline__ void cell_gradient(const Bufs& b, const Phys& ph, int
 				g[2 * q + 1] += s[q] / 2 * fy;
 			}
 		}
-		double isi = 1.0 / b.S[i];
+		double isi = rcp_dev(S);
 		for (int q = 0; q < 8; q++) g[q] *= isi;
 	}
+}
+
+template <bool MM, bool LSQ>
+__device__ __forceinline__ void cell_gradient(const Bufs& b, const Phys& ph, int i, Prim& pi, Prim* nb, double* g)
+{
+	pi = load_prim(b, i);
+	CellTop tp = load_top(b, i);
+	for (int k = 0; k < 3; k++) {
+		int j = tp.nb[k];
+		if (j >= 0) nb[k] = load_prim(b, j);
+		else nb[k] = ghost_of<MM>(b, ph, tp.f[k] >> 1, i, pi, pi);
+	}
+	double w[6];
+	ld6((LSQ ? b.lsqw : b.cfn) + 6 * (size_t)i, w);
+	gradient_sum<LSQ>(w, pi, nb, LSQ ? 0.0 : b.S[i], g);
 }
 
 template <bool MM, bool LSQ, bool LIM>
@@ -393,10 +469,9 @@ __global__ __launch_bounds__(BLOCK) void k_gradient(Bufs b, Phys ph)
 	double g[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 	if (i < b.nc) {
 		Prim pi;
-		int face[3];
 		Prim nb[3];
-		cell_gradient<MM, LSQ>(b, ph, i, pi, face, nb, g);
-		if (LIM) minmod_limit(b, i, face, pi, nb, g);
+		cell_gradient<MM, LSQ>(b, ph, i, pi, nb, g);
+		if (LIM) minmod_limit(b.cmid, b.nc, i, pi, nb, g);
 	}
 	store_records<8>(b.G, c0, min(BLOCK, b.nc - c0), g, lds);
 }
@@ -421,7 +496,7 @@ __device__ __forceinline__ void recon(Prim& q, const Bufs& b, int c, double dx, 
 __device__ __forceinline__ void grad_T_g(const double* g, const Prim& q, const MatV& m, double& tx, double& ty)
 {
 	// T = p / (r Rg), Rg = gR / M: grad T = (grad p - (p/r) grad r) / (r Rg)
-	double ir = 1.0 / q.r;
+	double ir = rcp_dev(q.r);
 	double pr = q.p * ir;
 	double s = ir * m.M * (1.0 / GAS_R);
 	tx = (g[2] - pr * g[0]) * s;
@@ -431,13 +506,13 @@ __device__ __forceinline__ void grad_T_g(const double* g, const Prim& q, const M
 // The lane pair's (f_gp1 + f_gp2) l/2 as the edge's 32-byte flux record: the
 // even lane adds its partner's flux to its own (the reference's order), the
 // odd lane the other way round (the same sums), and lane gp writes
-// components 2gp and 2gp+1, so the 64 lanes of a wave store 1 KB
-// contiguously
-__device__ __forceinline__ void store_edge_flux(double* F, int e, int gp, const double* f, const double* o, double hl)
+// components 2gp and 2gp+1 (out: its half of the record), so the 64 lanes of
+// a wave store 1 KB contiguously
+__device__ __forceinline__ void store_edge_flux(double* out, int gp, const double* f, const double* o, double hl)
 {
 	double a0 = gp ? f[2] + o[2] : f[0] + o[0];
 	double a1 = gp ? f[3] + o[3] : f[1] + o[1];
-	double* p = static_cast<double*>(__builtin_assume_aligned(F + 4 * (size_t)e + 2 * gp, 16));
+	double* p = static_cast<double*>(__builtin_assume_aligned(out, 16));
 	p[0] = a0 * hl;
 	p[1] = a1 * hl;
 }
@@ -483,23 +558,30 @@ struct EdgeShape<3> {  // 512 threads
 	static constexpr int NT = 512, WPE = 1;
 };
 constexpr int EDGE_SHAPES = 4;
+constexpr int FLUX_GODUNOV14 = 4;  // a kernel's exact Godunov flux at GAM = 1.4
 
 // One lane of an edge's pair from the primitives ps and gradients gs of the
-// cell cs it reconstructs (c2 for the second lane of an inner edge, c1
+// cell it reconstructs (c2 for the second lane of an inner edge, c1
 // otherwise) onward: reconstruction, ghost, viscous terms, numerical flux and
-// the pair's combined store.  Shared by the edge passes, so they give the
-// same bits.
-template <bool MM, int FLUX, bool VISC>
-__device__ __forceinline__ void edge_lane(const Bufs& b, const Phys& ph, int e, int gp, int c1, bool inner, int cs,
-                                          const Prim& ps, const double* gs, double nx, double ny)
+// the pair's combined store (out: this lane's half of the record).  (nx, ny), l and dl are the
+// edge's normal, length and this lane's record of edl, bound the boundary
+// (not inner), m1 and ms the materials of c1 and of this lane's cell.
+// Returns whether the Newton iteration hit its cap.  Shared by the edge
+// passes, so they give the same bits.
+// STASH: out is in LDS, and the viscous stress waits out the Riemann solve
+// there instead of in registers (four fewer; the Navier-Stokes stage kernel
+// is at its limit).
+template <int FLUX, bool VISC, bool STASH>
+__device__ __forceinline__ int edge_lane(const Phys& ph, int gp, bool inner, const Bound& bound, const MatV& m1,
+                                         const MatV& ms, const Prim& ps, const double* gs, double nx, double ny,
+                                         double l, const double* dl, double* out)
 {
 	// Each lane extrapolates its own cell to its own Gauss point (kept) and to
 	// the partner's (sent); on an inner edge the pair swaps the sent states,
 	// so lane 0 holds (c1, c2) at Gauss point 1 and lane 1 at Gauss point 2 --
 	// the same operations as each lane reconstructing both cells.  On a
 	// boundary both lanes reconstruct c1 and build the ghost from it.
-	double dl[4];  // this lane's record: offsets of cs at its own, then the partner's Gauss point
-	ld4(b.edl, 2 * (size_t)e + gp, dl);
+	// dl: offsets of this lane's cell at its own, then the partner's Gauss point
 	Prim keep = ps, send = ps, recv;
 	recon_g(keep, gs, dl[0], dl[1]);
 	recon_g(send, gs, dl[2], dl[3]);
@@ -513,7 +595,7 @@ __device__ __forceinline__ void edge_lane(const Bufs& b, const Phys& ph, int e, 
 		R = gp ? keep : recv;
 	} else {
 		L = keep;
-		R = ghost_of<MM>(b, ph, e, c1, L, ps);
+		R = ghost_at(bound, nx, ny, L, ps, m1);
 	}
 	// Viscous terms first (only sx, sy and the energy term stay live through
 	// the Riemann solve).  Face gradient = mean of the two cell gradients (the
@@ -523,10 +605,10 @@ __device__ __forceinline__ void edge_lane(const Bufs& b, const Phys& ph, int e, 
 	// the same means.
 	double sx = 0.0, sy = 0.0, ev = 0.0;
 	if (VISC) {
-		MatV m = mat_of<MM>(b, ph, c1);
+		const MatV& m = m1;
 		double own[6];
 		for (int q = 0; q < 4; q++) own[q] = gs[4 + q];  // ux uy vx vy
-		grad_T_g(gs, ps, mat_of<MM>(b, ph, cs), own[4], own[5]);
+		grad_T_g(gs, ps, ms, own[4], own[5]);
 		double oth[6];
 		for (int q = 0; q < 6; q++) oth[q] = pair_swap(own[q]);
 		double ux = own[0], uy = own[1], vx = own[2], vy = own[3], tx = own[4], ty = own[5];
@@ -546,22 +628,32 @@ __device__ __forceinline__ void edge_lane(const Bufs& b, const Phys& ph, int e, 
 		sy = txy * nx + tyy * ny;
 		double uf = 0.5 * (L.u + R.u), vf = 0.5 * (L.v + R.v);
 		ev = uf * sx + vf * sy + m.kc * (tx * nx + ty * ny);
+		if (STASH) {
+			volatile double* w = out;
+			w[0] = sx;
+			w[1] = sy;
+		}
 	}
 	double f[4];
 	int hit = 0;
-	if (FLUX == CFD2D_FLUX_LAX) flux_lax(f, L, R, nx, ny, ph.gam_flux);
-	else if (FLUX == CFD2D_FLUX_HLLC) flux_hllc(f, L, R, nx, ny, ph.gam_flux);
+	if (FLUX == CFD2D_FLUX_LAX) flux_lax(f, L, R, nx, ny, ph.gam_flux, ph.igm1);
+	else if (FLUX == CFD2D_FLUX_HLLC) flux_hllc(f, L, R, nx, ny, ph.gam_flux, ph.igm1);
 	else if (FLUX == CFD2D_FLUX_ROE) flux_roe(f, L, R, nx, ny, ph.gam_flux);
-	else flux_godunov(f, L, R, nx, ny, ph.rk, ph.max_newton, hit);
-	if (hit) atomicAdd(&b.err[0], 1ull);
+	else flux_godunov<FLUX == FLUX_GODUNOV14>(f, L, R, nx, ny, ph.rk, ph.max_newton, hit);
 	if (VISC) {
+		if (STASH) {
+			volatile double* w = out;
+			sx = w[0];
+			sy = w[1];
+		}
 		f[1] -= sx;
 		f[2] -= sy;
 		f[3] -= ev;
 	}
 	double o[4];
 	for (int q = 0; q < 4; q++) o[q] = pair_swap(f[q]);
-	store_edge_flux(b.F, e, gp, f, o, edge_geo(b, e)[2] * 0.5);
+	store_edge_flux(out, gp, f, o, l * 0.5);
+	return hit;
 }
 
 template <bool MM, int FLUX, bool VISC, int GR, int SHAPE = 0>
@@ -579,84 +671,45 @@ __global__ __attribute__((amdgpu_flat_work_group_size(1, EdgeShape<SHAPE>::NT),
 	double gs[8];                          // its gradients
 	Prim ps;                               // and primitives
 	if (GR) {
-		int face[3];
 		Prim nb[3];
-		cell_gradient<MM, GR == 1 || GR == 3>(b, ph, cs, ps, face, nb, gs);
-		if (GR >= 3) minmod_limit(b, cs, face, ps, nb, gs);
+		cell_gradient<MM, GR == 1 || GR == 3>(b, ph, cs, ps, nb, gs);
+		if (GR >= 3) minmod_limit(b.cmid, b.nc, cs, ps, nb, gs);
 	} else {
 		ps = load_prim(b, cs);
 		ld8(b.G, cs, gs);
 	}
-	edge_lane<MM, FLUX, VISC>(b, ph, e, gp, c1, inner, cs, ps, gs, nx, ny);
+	double dl[4];
+	ld4(b.edl, 2 * (size_t)e + gp, dl);
+	Bound bound{};
+	if (!inner) bound = load_bound(b, -c2 - 1);
+	if (edge_lane<FLUX, VISC, false>(ph, gp, inner, bound, mat_of<MM>(b, ph, c1), mat_of<MM>(b, ph, cs), ps, gs, nx, ny,
+	                          edge_geo(b, e)[2], dl, b.F + 4 * (size_t)e + 2 * gp))
+		atomicAdd(&b.err[0], 1ull);
 }
 
-// Tiled edge pass (fuse mode 2): one workgroup per tile of TILE_CELLS
-// consecutive cells.  The tile owns the edges whose c1 it holds -- a
-// contiguous edge range, since edges are numbered in c1 order -- and first
-// forms, once each, the gradients of every cell those edges read (its own
-// cells and the c2 cells beyond it) with the gradient pass's code, staging
-// primitives and gradients in LDS; then the lane pairs of its edges run
-// edge_lane from LDS.  A cell's gradient is formed by ~1.25 tiles instead of
-// by each of its three edges, and the edge lanes gather nothing but their
-// edge's own records.  The same bits as the other edge passes.
-constexpr int TILE_CELLS = 256;  // cells per tile (smaller when the staged set would not fit)
-constexpr int TILE_CAP = 384;    // staged cells per tile at most
-constexpr int TILE_ROW = 12;     // LDS doubles per staged cell: r, p, u, v, then the 8 gradients
-
-template <bool MM, int FLUX, bool VISC, int GR>
-__global__ __launch_bounds__(BLOCK) void k_edge_tile(Bufs b, Phys ph)
-{
-	__shared__ double stage[TILE_CAP * TILE_ROW];
-	int4 tl = reinterpret_cast<const int4*>(b.tiles)[xcd_block()];  // first staged cell, count, first edge, count
-	for (int k = threadIdx.x; k < tl.y; k += BLOCK) {
-		int c = b.tcell[tl.x + k];
-		Prim pi;
-		int face[3];
-		Prim nb[3];
-		double g[8];
-		cell_gradient<MM, GR == 1 || GR == 3>(b, ph, c, pi, face, nb, g);
-		if (GR >= 3) minmod_limit(b, c, face, pi, nb, g);
-		double* r = stage + TILE_ROW * k;
-		r[0] = pi.r;
-		r[1] = pi.p;
-		r[2] = pi.u;
-		r[3] = pi.v;
-		for (int q = 0; q < 8; q++) r[4 + q] = g[q];
-	}
-	__syncthreads();
-	// lane pairs (t, t + 1) stay together: BLOCK is even
-	for (int t = threadIdx.x; t < 2 * tl.w; t += BLOCK) {
-		int e = tl.z + (t >> 1), gp = t & 1;
-		int2 ce = edge_cells(b, e);
-		bool inner = ce.y >= 0;
-		bool second = gp == 1 && inner;
-		unsigned sl = b.eslot[e];
-		const double* r = stage + TILE_ROW * (int)(second ? sl >> 16 : sl & 0xffffu);
-		Prim ps{r[0], r[1], r[2], r[3]};
-		double gs[8];
-		for (int q = 0; q < 8; q++) gs[q] = r[4 + q];
-		edge_lane<MM, FLUX, VISC>(b, ph, e, gp, ce.x, inner, second ? ce.y : ce.x, ps, gs, edge_geo(b, e)[0],
-		                          edge_geo(b, e)[1]);
-	}
-}
-
-// residual of cell i: -F on c1's side, +F on c2's, ascending edge order
-// (the scatter of fvm_tvd.cpp:353-363 seen from the cell); an edge's flux is
-// one 32-byte record, two 16-byte loads
-__device__ __forceinline__ void gather_residual(const Bufs& b, int i, double* r)
+// residual of a cell from the flux records of its faces fs (get reads one):
+// -F on c1's side, +F on c2's, ascending edge order (the scatter of fvm_tvd.cpp:353-363
+// seen from the cell); an edge's flux is one 32-byte record, two 16-byte loads
+template <typename Get>
+__device__ __forceinline__ void sum_fluxes(Get get, const int* fs, double* r)
 {
 	r[0] = r[1] = r[2] = r[3] = 0.0;
-	int4 fc = load_faces(b, i);
-	int fs[3] = {fc.x, fc.y, fc.z};
 	for (int k = 0; k < 3; k++) {
 		int f = fs[k];
 		double v[4];
-		ld4(b.F, f >> 1, v);
+		get(f >> 1, v);
 		if (f & 1)
 			for (int q = 0; q < 4; q++) r[q] += v[q];
 		else
 			for (int q = 0; q < 4; q++) r[q] -= v[q];
 	}
+}
+
+__device__ __forceinline__ void gather_residual(const Bufs& b, int i, double* r)
+{
+	int4 fc = load_faces(b, i);
+	int fs[3] = {fc.x, fc.y, fc.z};
+	sum_fluxes([&](int e, double* v) { ld4(b.F, e, v); }, fs, r);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_residual(Bufs b)
@@ -676,25 +729,89 @@ enum { UPD_FIRST = 0, UPD_RK2_LAST = 2, UPD_RK3_MID = 3, UPD_RK3_LAST = 4 };
 // non-temporally (NT) so that they do not evict the primitives, fluxes and
 // geometry that the next edge pass gathers; a case that fits the cache
 // keeps them cached.  The values are the same either way.
-template <bool NT>
-__device__ __forceinline__ double ld_state(const double* p)
+__device__ __forceinline__ double ld_state(const double* p, bool nt)
 {
-	if (NT) return __builtin_nontemporal_load(p);
+	if (nt) return __builtin_nontemporal_load(p);
 	return *p;
 }
 
-template <bool NT>
-__device__ __forceinline__ void st_state(double* p, double v)
+__device__ __forceinline__ void st_state(double* p, double v, bool nt)
 {
-	if (NT) __builtin_nontemporal_store(v, p);
+	if (nt) __builtin_nontemporal_store(v, p);
 	else *p = v;
 }
 
-// Update pass (fvm_tvd.cpp:366-374, 419-447): LIM-flagged cells stay frozen;
-// the last stage forms the RK combination, refreshes the primitives and sets
-// the bound flags (clamped values are not written back, 439-446).  The stage
-// reads its input from b.U and the step-start state from b.U0 and writes
-// b.Un; launch_update points them so that the step-start state is never
+// What one cell's update reads besides its residual: its flags, the stage's
+// input state (b.U), the step-start state (b.U0, not in the first stage) and
+// tau / S
+struct CellIn {
+	unsigned fl;
+	double u[4], u0[4], dts;
+};
+
+__device__ __forceinline__ CellIn load_cell(const Bufs& b, int mode, bool nt, int i)
+{
+	CellIn c;
+	size_t n = b.nc;
+	c.fl = b.flags[i];
+	for (int q = 0; q < 4; q++) c.u[q] = ld_state(&b.U[q * n + i], nt);
+	for (int q = 0; q < 4; q++) c.u0[q] = mode != UPD_FIRST ? ld_state(&b.U0[q * n + i], nt) : 0.0;
+	c.dts = b.dtS[i];
+	return c;
+}
+
+// One cell's update (fvm_tvd.cpp:366-374, 419-447): LIM-flagged cells stay
+// frozen; the last stage forms the RK combination and sets the bound flags
+// (clamped values are not written back, 439-446).  Writes b.Un; res(r) gives
+// the residual of a cell that is not frozen.  pv (if given) takes the new
+// primitives; the result is whether the cell is LIM-flagged.
+template <bool MM, typename Res>
+__device__ __forceinline__ int update_cell(const Bufs& b, const Phys& ph, int mode, bool nt, int i, const CellIn& c,
+                                           Res res, double* pv)
+{
+	size_t n = b.nc;
+	if (c.fl & 0x2u) {
+		if (mode != UPD_RK2_LAST && mode != UPD_RK3_LAST && b.Un != b.U)  // a frozen cell's state still moves on
+			for (int q = 0; q < 4; q++) st_state(&b.Un[q * n + i], c.u[q], nt);
+		if (pv) ld4(b.P, i, pv);  // its primitives unchanged
+		return 1;
+	}
+	double r[4], u[4];
+	res(r);
+	for (int q = 0; q < 4; q++) {
+		double t = c.u[q] + c.dts * r[q];
+		if (mode == UPD_FIRST) u[q] = t;
+		else if (mode == UPD_RK2_LAST) u[q] = 0.5 * (c.u0[q] + t);
+		else if (mode == UPD_RK3_MID) u[q] = 0.75 * c.u0[q] + 0.25 * t;
+		else u[q] = (1.0 / 3.0) * c.u0[q] + (2.0 / 3.0) * t;
+	}
+	bool finite = true;
+	for (int q = 0; q < 4; q++) {
+		st_state(&b.Un[q * n + i], u[q], nt);
+		finite = finite && isfinite(u[q]);
+	}
+	if (!finite) atomicAdd(&b.err[1], 1ull);
+	MatV m = mat_of<MM>(b, ph, i);
+	Prim p = cons_to_prim(u[0], u[1], u[2], u[3], m);
+	if (pv) {
+		pv[0] = p.r;
+		pv[1] = p.p;
+		pv[2] = p.u;
+		pv[3] = p.v;
+	}
+	if (mode == UPD_RK2_LAST || mode == UPD_RK3_LAST) {
+		bool out = p.r < ph.ro_min || p.r > ph.ro_max || p.p < ph.p_min || p.p > ph.p_max || fabs(p.u) > ph.u_max ||
+		           fabs(p.v) > ph.u_max;
+		if (out) {
+			b.flags[i] = c.fl | 0x2u;
+			return 1;
+		}
+	}
+	return 0;
+}
+
+// Update pass: update_cell for every cell behind an edge pass's fluxes;
+// launch_update points its buffers so that the step-start state is never
 // copied (the reference's U_old copy, 318-321).  NT: see ld_state.  REC
 // (adjoint recording behind an edge pass that forms its own gradients, where
 // the stage's input primitives b.P and its output b.Po are separate slots):
@@ -713,62 +830,18 @@ __global__ __launch_bounds__(BLOCK) void k_update(Bufs b, Phys ph)
 		double g[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 		if (i < b.nc) {
 			Prim pi;
-			int face[3];
 			Prim nb[3];
-			if (b.lsqw) cell_gradient<MM, true>(b, ph, i, pi, face, nb, g);
-			else cell_gradient<MM, false>(b, ph, i, pi, face, nb, g);
+			if (b.lsqw) cell_gradient<MM, true>(b, ph, i, pi, nb, g);
+			else cell_gradient<MM, false>(b, ph, i, pi, nb, g);
 		}
 		// read only by the reverse sweep, many stages later: kept out of the caches
 		store_records<8, true>(b.G, lb * BLOCK, min(BLOCK, b.nc - lb * BLOCK), g, lds);
 		__syncthreads();  // lds is reused below
 	}
 	double pv[4] = {0.0, 0.0, 0.0, 0.0};  // primitives written for this cell
-	if (i < b.nc) {
-		size_t n = b.nc;
-		unsigned fl = b.flags[i];
-		bool lim = (fl & 0x2u) != 0;
-		double u[4], u0[4];
-		for (int q = 0; q < 4; q++) u[q] = ld_state<NT>(&b.U[q * n + i]);
-		if (MODE == UPD_FIRST && lim)  // a frozen cell's state still moves to the stage buffer
-			for (int q = 0; q < 4; q++) st_state<NT>(&b.Un[q * n + i], u[q]);
-		if (!lim) {
-			double r[4];
-			gather_residual(b, i, r);
-			double cfl = b.dtS[i];
-			if (MODE != UPD_FIRST)
-				for (int q = 0; q < 4; q++) u0[q] = ld_state<NT>(&b.U0[q * n + i]);
-			for (int q = 0; q < 4; q++) {
-				double t = u[q] + cfl * r[q];
-				if (MODE == UPD_FIRST) u[q] = t;
-				else if (MODE == UPD_RK2_LAST) u[q] = 0.5 * (u0[q] + t);
-				else if (MODE == UPD_RK3_MID) u[q] = 0.75 * u0[q] + 0.25 * t;
-				else u[q] = (1.0 / 3.0) * u0[q] + (2.0 / 3.0) * t;
-			}
-			bool finite = true;
-			for (int q = 0; q < 4; q++) {
-				st_state<NT>(&b.Un[q * n + i], u[q]);
-				finite = finite && isfinite(u[q]);
-			}
-			if (!finite) atomicAdd(&b.err[1], 1ull);
-			MatV m = mat_of<MM>(b, ph, i);
-			Prim p = cons_to_prim(u[0], u[1], u[2], u[3], m);
-			pv[0] = p.r;
-			pv[1] = p.p;
-			pv[2] = p.u;
-			pv[3] = p.v;
-			if (MODE == UPD_RK2_LAST || MODE == UPD_RK3_LAST) {
-				bool out = p.r < ph.ro_min || p.r > ph.ro_max || p.p < ph.p_min || p.p > ph.p_max ||
-				           fabs(p.u) > ph.u_max || fabs(p.v) > ph.u_max;
-				if (out) {
-					fl |= 0x2u;
-					b.flags[i] = fl;
-				}
-			}
-		} else {
-			ld4(b.P, i, pv);  // frozen cell: its primitives unchanged
-		}
-		flagged = (fl & 0x2u) != 0;
-	}
+	if (i < b.nc)
+		flagged = update_cell<MM>(b, ph, MODE, NT, i, load_cell(b, MODE, NT, i),
+		                          [&](double* r) { gather_residual(b, i, r); }, pv);
 	store_records<4>(b.Po, lb * BLOCK, min(BLOCK, b.nc - lb * BLOCK), pv, lds);
 	if (MODE == UPD_RK2_LAST || MODE == UPD_RK3_LAST) {
 		int any = __syncthreads_or(flagged);
@@ -779,6 +852,290 @@ __global__ __launch_bounds__(BLOCK) void k_update(Bufs b, Phys ph)
 				atomicOr(b.anyflag + 1, 1);
 			}
 		}
+	}
+}
+
+// FVM_TVD::calcTimeStep (src/methods/fvm_tvd.cpp:216-240): local step
+// CFL*S/max(|u|+c, |v|+c) with the cell area S (spectral variant:
+// 2*CFL*S / sum_f lambda_f l_f); steady runs keep it per cell.  nb: the
+// neighbours' states, ghosts on a boundary (spectral variant only).
+template <bool MM>
+__device__ __forceinline__ double local_step(const Bufs& b, const Phys& ph, int i, const Prim& p, const Prim* nb)
+{
+	MatV m = mat_of<MM>(b, ph, i);
+	double cz = sqrt(m.gam * p.p / p.r);
+	double S = b.S[i];
+	if (ph.cfl_mode == CFD2D_CFL_SPECTRAL) {
+		double li = sqrt(p.u * p.u + p.v * p.v) + cz;
+		double sum = 0.0;
+		CellTop tp = load_top(b, i);
+		for (int k = 0; k < 3; k++) {
+			const Prim& q = nb[k];
+			MatV mj = tp.nb[k] >= 0 ? mat_of<MM>(b, ph, tp.nb[k]) : m;
+			double czj = sqrt(mj.gam * q.p / q.r);
+			double lj = sqrt(q.u * q.u + q.v * q.v) + czj;
+			sum += 0.5 * (li + lj) * edge_geo(b, tp.f[k] >> 1)[2];
+		}
+		return 2.0 * ph.cfl * S / sum;
+	}
+	double a = fabs(p.u) + cz, c = fabs(p.v) + cz;
+	return ph.cfl * S / (a > c ? a : c);
+}
+
+// One whole RK stage by tiles: a workgroup owns a group of cells that lie
+// together (build_tiles) and stages them and every cell across their faces.
+// From the conserved state of these and of the cells around them it forms
+// primitives in LDS; each staged cell's gradient (limited if asked) once, by
+// one lane, with the gradient pass's code; then the lane pairs of every edge
+// of an own cell run edge_lane from LDS and leave the edge's flux there; then
+// the own cells are updated with the update pass's code.  Neither primitives,
+// gradients nor fluxes touch memory, and a stage is one launch; an edge
+// between two tiles is evaluated by both (the same bits) and a cell next to
+// another tile has its primitives and gradient formed again.  The stage reads
+// b.U around its tile, so it may not write there: it writes b.Un.  store_g
+// (adjoint recording): the own cells' input primitives and gradients go to
+// b.P and b.G.  Steady runs: the first stage sets the cells' time steps.
+//
+// Everything a tile reads except the state sits at addresses that follow
+// from the block index, so the state is one dependent load away from the
+// launch.
+//
+// On 2 M cells (Navier-Stokes, LSQ, exact Godunov) a stage takes 190 us, the
+// edge and update passes it replaces 174 + 76 us, and moves 0.72 GB of memory
+// instead of 1.09.  64 % of its vector issue slots are filled: what bounds it
+// is FP64 issue, with the phases of a tile (load, gradients, edges, update)
+// overlapped only across the five workgroups of a compute unit.  On 8 000
+// cells a stage takes 8 us against 6.6 + 4.
+//
+// Tile sizes: an own cell has about 1.6 edges in its tile, so 256 edges are
+// two turns of the 256 lanes through the edge loop, and the LDS of such a
+// tile (29 KB) leaves room for five workgroups per compute unit, which the
+// edge loop's registers (96) allow.  The limiter and the general-gamma
+// Riemann solver spill at 96 registers: four workgroups, and the limiter's
+// contexts have the larger tiles that fit those.  2 M cells, Navier-Stokes,
+// per step: 256-edge tiles and five workgroups 0.57 ms, 352 and four 0.60,
+// 192-lane workgroups 0.59, 512-lane 0.60, 320-lane 0.72 (spilled).  64
+// limited channels: 352 edges and four workgroups 0.231 ms, 256 and four
+// 0.239, 256 and five 0.246.
+template <bool LIM>
+struct StageShape {
+	static constexpr int ALL = 256;    // cells per tile at most
+	static constexpr int CELLS = 208;  // staged cells at most: one per lane
+	static constexpr int EDGES = 256;  // edges at most
+	static constexpr int WAVES = 5;    // workgroups per compute unit, waves per SIMD
+};
+template <>
+struct StageShape<true> {
+	static constexpr int ALL = 320, CELLS = 256, EDGES = 352, WAVES = 4;
+};
+constexpr int STAGE_THREADS = 256;
+
+struct StageArgs {
+	Bufs b;
+	Phys ph;
+	int mode, nt;
+};
+
+// The kernel's arguments read again from the kernel-argument segment.  Each
+// part of k_stage takes its own copy: held in scalar registers from the
+// kernel's start, the pointers of the later parts and the Riemann solver's
+// constants do not fit beside each other and are moved to vector lanes and
+// back inside the edge loop (124 of 709 vector instructions per wave).
+__device__ __forceinline__ StageArgs args_again(const StageArgs& a)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+	auto* p = (const __attribute__((address_space(4))) StageArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+	asm volatile("" : "+s"(p));  // not the same pointer, as far as the compiler knows
+	return *p;
+#else
+	return a;
+#endif
+}
+
+// 16-byte pieces in LDS: every record is kept as pieces of two doubles, each
+// piece number in an array of its own, so that neighbouring lanes' reads of
+// neighbouring records fall into different banks
+__device__ __forceinline__ void ld2(const double (*a)[2], int i, double* v)
+{
+	const double* p = static_cast<const double*>(__builtin_assume_aligned(a[i], 16));
+	v[0] = p[0];
+	v[1] = p[1];
+}
+
+__device__ __forceinline__ void st2(double (*a)[2], int i, const double* v)
+{
+	double* p = static_cast<double*>(__builtin_assume_aligned(a[i], 16));
+	p[0] = v[0];
+	p[1] = v[1];
+}
+
+template <bool MM, int FLUX, bool VISC, int GR>
+__global__ __attribute__((amdgpu_flat_work_group_size(1, STAGE_THREADS),
+                          amdgpu_waves_per_eu(FLUX == CFD2D_FLUX_GODUNOV ? 4 : StageShape<GR >= 3>::WAVES))) void
+k_stage(StageArgs args)
+{
+	using Shape = StageShape<GR >= 3>;
+	__shared__ __align__(16) double prim[2][Shape::ALL][2];    // (r, p), (u, v)
+	__shared__ __align__(16) double grad[4][Shape::CELLS][2];  // of r, p, u, v
+	// an edge's geometry record, then, written by its lanes when they are done
+	// with that, its flux record
+	__shared__ __align__(16) double flux[2][Shape::EDGES][2];
+	auto prim_of = [&](int i) {
+		double v[4];
+		ld2(prim[0], i, v);
+		ld2(prim[1], i, v + 2);
+		return Prim{v[0], v[1], v[2], v[3]};
+	};
+	int tile = xcd_block(), t = threadIdx.x;
+	int4 hd = args.b.thead[tile];
+	{
+		const StageArgs a = args_again(args);
+		const Bufs& b = a.b;
+		const int* cells = b.tcell + (size_t)tile * b.tall;
+		const double* geo = b.tgeo + 4 * (size_t)tile * b.tec;
+		for (int k = t; k < 2 * hd.w; k += b.tthreads) {
+			const double* g = static_cast<const double*>(__builtin_assume_aligned(geo + 2 * k, 16));
+			double v[2] = {g[0], g[1]};
+			st2(flux[k & 1], k >> 1, v);
+		}
+		for (int k = t; k < hd.z; k += b.tthreads) {
+			int c = cells[k];
+			double u[4];
+			lda4(b.U, b.nc, c, u);
+			Prim p = cons_to_prim(u[0], u[1], u[2], u[3], mat_of<MM>(b, a.ph, c));
+			double v[4] = {p.r, p.p, p.u, p.v};
+			st2(prim[0], k, v);
+			st2(prim[1], k, v + 2);
+		}
+	}
+	__syncthreads();
+	if (t < hd.y) {
+		const StageArgs a = args_again(args);
+		const Bufs& b = a.b;
+		const Phys& ph = a.ph;
+		size_t cb = (size_t)tile * b.tsc;
+		int4 rc = b.trec[cb + t];
+		int nj[3] = {rc.x, rc.y, rc.z};
+		Prim pi = prim_of(t);
+		Prim nb[3];
+		double g[8], w[6];
+		ld6(b.tw + 6 * (cb + t), w);
+		for (int k = 0; k < 3; k++) {
+			if (nj[k] >= 0) nb[k] = prim_of(nj[k]);
+			else nb[k] = ghost_of<MM>(b, ph, -1 - nj[k], rc.w, pi, pi);
+		}
+		gradient_sum<GR == 1 || GR == 3>(w, pi, nb, GR == 1 || GR == 3 ? 0.0 : b.S[rc.w], g);
+		if (GR >= 3) minmod_limit(b.tcmid + 4 * cb, b.tsc, t, pi, nb, g);
+		for (int q = 0; q < 4; q++) st2(grad[q], t, g + 2 * q);
+		if (a.mode == UPD_FIRST && ph.steady && t < hd.x) {
+			double loc = local_step<MM>(b, ph, rc.w, pi, nb);
+			b.loc[rc.w] = loc;
+			b.dtS[rc.w] = loc / b.S[rc.w];
+		}
+	}
+	__syncthreads();
+	if (args_again(args).ph.store_g) {
+		const StageArgs a = args_again(args);
+		const Bufs& b = a.b;
+		// read only by the reverse sweep, many stages later: kept out of the caches
+		for (int k = t; k < 6 * hd.x; k += b.tthreads) {
+			bool g = k < 4 * hd.x;
+			int j = g ? k : k - 4 * hd.x, i = g ? j >> 2 : j >> 1, q = j & (g ? 3 : 1);
+			int c = b.tcell[(size_t)tile * b.tall + i];
+			double v[2];
+			ld2(g ? grad[q] : prim[q], i, v);
+			double* o = static_cast<double*>(
+			    __builtin_assume_aligned((g ? b.G + 8 * (size_t)c : b.P + 4 * (size_t)c) + 2 * q, 16));
+			__builtin_nontemporal_store(v[0], o);
+			__builtin_nontemporal_store(v[1], o + 1);
+		}
+	}
+	// lane pairs (t, t + 1) stay together: the workgroup size is even.  A wave
+	// past the last edge leaves; where a whole workgroup meets at each lane
+	// exchange (a host build of these kernels), its lanes repeat the last edge.
+	{
+		const StageArgs a = args_again(args);
+		const Bufs& b = a.b;
+		const Phys& ph = a.ph;
+		int gp = t & 1;
+		for (int w0 = 0; w0 < 2 * hd.w; w0 += b.tthreads) {
+			bool live = w0 + t < 2 * hd.w;
+#ifdef __HIP_DEVICE_COMPILE__
+			if (!live) break;
+#endif
+			int el = live ? (w0 + t) >> 1 : hd.w - 1;
+			const double* mid = static_cast<const double*>(
+			    __builtin_assume_aligned(b.tmid + 4 * ((size_t)tile * b.tec + el) + 2 * gp, 16));
+			double mx = mid[0], my = mid[1];
+			double n[2], sl[2];
+			ld2(flux[0], el, n);
+			ld2(flux[1], el, sl);
+			int2 pk = __builtin_bit_cast(int2, sl[1]);
+			double dl[4];
+			edge_offset(mx, my, n[0], n[1], sl[0], gp, dl);
+			edge_offset(mx, my, n[0], n[1], sl[0], 1 - gp, dl + 2);
+			bool inner = pk.y >= 0;
+			Bound bound{};
+			if (!inner) bound = load_bound(b, -1 - pk.y);
+			int cs = gp == 1 && inner ? pk.y : pk.x >> 1;
+			Prim ps = prim_of(cs);
+			double gs[8];
+			for (int q = 0; q < 4; q++) ld2(grad[q], cs, gs + 2 * q);
+			MatV m1 = ph.m0, ms = ph.m0;
+			if (MM) {
+				const int4* rec = b.trec + (size_t)tile * b.tsc;
+				m1 = mat_of<MM>(b, ph, rec[pk.x >> 1].w);
+				ms = mat_of<MM>(b, ph, rec[cs].w);
+			}
+			int hit = edge_lane<FLUX, VISC, true>(ph, gp, inner, bound, m1, ms, ps, gs, n[0], n[1], fabs(sl[0]), dl,
+			                                      flux[gp][el]);
+			if (hit && live && (pk.x & 1)) atomicAdd(&b.err[0], 1ull);
+		}
+	}
+	__syncthreads();
+	if (t < hd.x) {
+		const StageArgs a = args_again(args);
+		const Bufs& b = a.b;
+		int i = b.tcell[(size_t)tile * b.tall + t];
+		int2 fc = b.tface[(size_t)tile * b.tsc + t];
+		int fs[3] = {fc.x & 0xffff, (int)((unsigned)fc.x >> 16), fc.y};
+		auto get = [&](int e, double* v) {
+			ld2(flux[0], e, v);
+			ld2(flux[1], e, v + 2);
+		};
+		int flagged = update_cell<MM>(b, a.ph, a.mode, a.nt != 0, i, load_cell(b, a.mode, a.nt != 0, i),
+		                              [&](double* r) { sum_fluxes(get, fs, r); }, nullptr);
+		if (flagged && (a.mode == UPD_RK2_LAST || a.mode == UPD_RK3_LAST)) {
+			// cleared by the remediation that this raises
+			b.blockflag[i / BLOCK] = 1;
+			b.anyflag[0] = 1;
+			b.anyflag[1] = 1;
+		}
+	}
+}
+
+// A tile's static arrays from the context's own (build_tiles gives the cells
+// and, in tgeo's place, its edges): weights, limiter offsets, edge geometry
+__global__ __launch_bounds__(BLOCK) void k_fill_tiles(Bufs b, const double* w, const int4* edges,
+                                                      const double* esl, const double* emid)
+{
+	int tile = blockIdx.x;
+	int4 hd = b.thead[tile];
+	size_t cb = (size_t)tile * b.tsc, eb = (size_t)tile * b.tec;
+	for (int t = threadIdx.x; t < hd.y; t += BLOCK) {
+		int c = b.trec[cb + t].w;
+		for (int q = 0; q < 6; q++) b.tw[6 * (cb + t) + q] = w[6 * (size_t)c + q];
+		if (b.tcmid)
+			for (int q = 0; q < 4; q++) b.tcmid[4 * cb + (size_t)q * b.tsc + t] = b.cmid[(size_t)q * b.nc + c];
+	}
+	for (int t = threadIdx.x; t < hd.w; t += BLOCK) {
+		int4 ed = edges[eb + t];
+		const double* geo = edge_geo(b, ed.x);
+		b.tgeo[4 * (eb + t)] = geo[0];
+		b.tgeo[4 * (eb + t) + 1] = geo[1];
+		b.tgeo[4 * (eb + t) + 2] = esl[ed.x];
+		*reinterpret_cast<int2*>(b.tgeo + 4 * (eb + t) + 3) = edge_pack(ed.y, ed.z, ed.w != 0);
+		for (int q = 0; q < 4; q++) b.tmid[4 * (eb + t) + q] = emid[4 * (size_t)ed.x + q];
 	}
 }
 
@@ -873,53 +1230,28 @@ __global__ __launch_bounds__(BLOCK) void k_remediate(Bufs b, Phys ph)
 				MatV m = mat_of<MM>(b, ph, i);
 				store_prim(b, i, cons_to_prim(u[0], u[1], u[2], u[3], m));
 			}
+			if (tid == 0) b.blockflag[bb] = 0;  // set again by the next step that leaves a LIM cell here
 			__syncthreads();  // the next block gathers what this one stored
 		}
 	}
 	if (tid == 0) *b.anyflag = 0;
 }
 
-// FVM_TVD::calcTimeStep (src/methods/fvm_tvd.cpp:216-240): local step
-// CFL*S/max(|u|+c, |v|+c) with the cell area S (spectral variant:
-// 2*CFL*S / sum_f lambda_f l_f); steady runs keep it per cell.
 template <bool MM>
 __global__ __launch_bounds__(BLOCK) void k_tau(Bufs b, Phys ph)
 {
 	int i = xcd_block() * BLOCK + threadIdx.x;
 	if (i >= b.nc) return;
 	Prim p = load_prim(b, i);
-	MatV m = mat_of<MM>(b, ph, i);
-	double cz = sqrt(m.gam * p.p / p.r);
-	double S = b.S[i];
-	double loc;
+	Prim nb[3];
 	if (ph.cfl_mode == CFD2D_CFL_SPECTRAL) {
-		double li = sqrt(p.u * p.u + p.v * p.v) + cz;
-		double sum = 0.0;
 		CellTop tp = load_top(b, i);
-		for (int k = 0; k < 3; k++) {
-			int f = tp.f[k];
-			int e = f >> 1;
-			int j = tp.nb[k];
-			Prim q;
-			double czj;
-			if (j >= 0) {
-				q = load_prim(b, j);
-				MatV mj = mat_of<MM>(b, ph, j);
-				czj = sqrt(mj.gam * q.p / q.r);
-			} else {
-				q = ghost_of<MM>(b, ph, e, i, p, p);
-				czj = sqrt(m.gam * q.p / q.r);
-			}
-			double lj = sqrt(q.u * q.u + q.v * q.v) + czj;
-			sum += 0.5 * (li + lj) * edge_geo(b, e)[2];
-		}
-		loc = 2.0 * ph.cfl * S / sum;
-	} else {
-		double a = fabs(p.u) + cz, c = fabs(p.v) + cz;
-		loc = ph.cfl * S / (a > c ? a : c);
+		for (int k = 0; k < 3; k++)
+			nb[k] = tp.nb[k] >= 0 ? load_prim(b, tp.nb[k]) : ghost_of<MM>(b, ph, tp.f[k] >> 1, i, p, p);
 	}
+	double loc = local_step<MM>(b, ph, i, p, nb);
 	b.loc[i] = loc;
-	if (ph.steady) b.dtS[i] = loc / S;
+	if (ph.steady) b.dtS[i] = loc / b.S[i];
 }
 
 }  // namespace
@@ -934,6 +1266,8 @@ struct cfd2d_ctx {
 	Bufs b{};
 	hipStream_t st = nullptr;
 	std::vector<double> hS;
+	bool prim_stale = false;  // b.P is not U's (refresh_prim)
+	bool c1_order = true;  // edges in ascending order of c1
 	std::vector<int> hc1;  // edge c1, length, normal (host copies for the force integrals)
 	std::vector<double> hel, hnx, hny;
 	std::vector<int> case_off;
@@ -941,9 +1275,8 @@ struct cfd2d_ctx {
 	// timing
 	bool timing = false;
 	unsigned timing_mask = ~0u;  // kernel ids (bit CFD2D_K_*) that get events
-	int fuse_mode = -1;          // 1: the edge pass forms the gradients, 2: the tiled edge
-	                             // pass does, 0: a separate gradient pass, -1: 1 without
-	                             // a limiter, 0 with one
+	int fuse_mode = -1;          // -1, 2: a stage is one kernel, 1: the edge pass forms the
+	                             // gradients, 0: a separate gradient pass does
 	bool prefer_graph = false;   // cfd2d_step replays a recorded step (chosen by cfd2d_autotune)
 	int edge_shape = 0;          // launch shape of the edge pass (EdgeShape; chosen by cfd2d_autotune)
 	int stream_mode = -1;        // update pass reads/writes the state non-temporally: 1 yes,
@@ -996,6 +1329,7 @@ struct cfd2d_ctx {
 namespace {
 
 constexpr int EV_POOL = 8192;
+constexpr int CU_COUNT = 256;  // compute units
 constexpr size_t LLC_BYTES = (size_t)256 << 20;  // MI355X Infinity Cache (last-level, shared by the XCDs)
 
 int hip_fail(hipError_t e, const char* what)
@@ -1032,6 +1366,15 @@ int upload(cfd2d_ctx* c, T** p, const std::vector<T>& v)
 }
 
 int grid_of(int n) { return (n + BLOCK - 1) / BLOCK; }
+
+// Own cells per tile at most: small meshes are cut finer, into four tiles
+// (what a compute unit holds at once) for every compute unit, as long as a
+// tile keeps 40 cells; below, the cells and edges formed twice outweigh it
+int tile_cells(int nc) { return std::max(40, (nc + 4 * CU_COUNT - 1) / (4 * CU_COUNT)); }
+
+// Threads per tile: a lane per staged cell, and for small tiles a lane per
+// edge and Gauss point
+int tile_threads(int sc, int ec) { return std::min((std::max(sc, 2 * ec) + 63) / 64 * 64, STAGE_THREADS); }
 
 void rec_start(cfd2d_ctx* c, int k)
 {
@@ -1080,6 +1423,9 @@ void harvest(cfd2d_ctx* c)
 		hipLaunchKernelGGL(kern, dim3(grid_of(n)), dim3(BLOCK), 0, (c)->st, __VA_ARGS__);   \
 		rec_stop(c);                                                                        \
 	} while (0)
+
+// whether a stage is one launch of the stage kernel (fuse modes -1 and 2)
+bool stage_path(const cfd2d_ctx* c) { return c->fuse_mode < 0 || c->fuse_mode == 2; }
 
 template <bool MM>
 void launch_prim(cfd2d_ctx* c)
@@ -1142,53 +1488,18 @@ void launch_edge(cfd2d_ctx* c)
 	else launch_edge_v<MM, false, 0>(c);
 }
 
-// gradient + edge passes of one stage: by default the edge pass forms the
-// gradients itself without a limiter (nothing reads the stored gradients
-// afterwards) and a separate pass forms them with one (three limiter
-// evaluations per cell cost more than the pass they save on large meshes);
-// cfd2d_fuse_gradient and cfd2d_autotune change the choice
-template <bool MM, bool VISC, int GR>
-void launch_edge_tile(cfd2d_ctx* c)
-{
-	dim3 g(c->b.ntiles), blk(BLOCK);
-	rec_start(c, CFD2D_K_EDGE_FLUX);
-	switch (c->p.flux) {
-	case CFD2D_FLUX_LAX: hipLaunchKernelGGL((k_edge_tile<MM, CFD2D_FLUX_LAX, VISC, GR>), g, blk, 0, c->st, c->b, c->ph); break;
-	case CFD2D_FLUX_HLLC: hipLaunchKernelGGL((k_edge_tile<MM, CFD2D_FLUX_HLLC, VISC, GR>), g, blk, 0, c->st, c->b, c->ph); break;
-	case CFD2D_FLUX_ROE: hipLaunchKernelGGL((k_edge_tile<MM, CFD2D_FLUX_ROE, VISC, GR>), g, blk, 0, c->st, c->b, c->ph); break;
-	default: hipLaunchKernelGGL((k_edge_tile<MM, CFD2D_FLUX_GODUNOV, VISC, GR>), g, blk, 0, c->st, c->b, c->ph); break;
-	}
-	rec_stop(c);
-}
-
-template <bool MM, bool VISC>
-void launch_edge_tiled(cfd2d_ctx* c, int gr)
-{
-	switch (gr) {
-	case 1: launch_edge_tile<MM, VISC, 1>(c); break;
-	case 2: launch_edge_tile<MM, VISC, 2>(c); break;
-	case 3: launch_edge_tile<MM, VISC, 3>(c); break;
-	default: launch_edge_tile<MM, VISC, 4>(c); break;
-	}
-}
-
+// gradient + edge passes of one stage (fuse modes 0 and 1)
 template <bool MM>
 void launch_gradient_edge(cfd2d_ctx* c)
 {
 	bool lim = c->p.limiter != CFD2D_LIMITER_NONE;
-	bool fuse = c->fuse_mode < 0 ? !lim : c->fuse_mode != 0;
-	if (!fuse) {
+	if (c->fuse_mode == 0) {
 		launch_gradient<MM>(c);
 		launch_edge<MM>(c);
 		return;
 	}
 	bool lsq = c->p.gradient == CFD2D_GRAD_LSQ;
 	int gr = (lsq ? 1 : 2) + (lim ? 2 : 0);
-	if (c->fuse_mode == 2 && c->b.ntiles > 0) {
-		if (c->p.viscous) launch_edge_tiled<MM, true>(c, gr);
-		else launch_edge_tiled<MM, false>(c, gr);
-		return;
-	}
 	if (c->p.viscous) {
 		switch (gr) {
 		case 1: launch_edge_v<MM, true, 1>(c); break;
@@ -1241,23 +1552,66 @@ void launch_update(cfd2d_ctx* c, int mode)
 	else launch_update_nt<MM, false, false>(c, mode, b);
 }
 
+template <bool MM, int FLUX, bool VISC>
+void launch_stage_f(cfd2d_ctx* c, const Bufs& b, int mode, int nt)
+{
+	dim3 g(b.ntiles), blk(b.tthreads);
+	StageArgs a{b, c->ph, mode, nt};
+	int gr = (c->p.gradient == CFD2D_GRAD_LSQ ? 1 : 2) + (c->p.limiter != CFD2D_LIMITER_NONE ? 2 : 0);
+	rec_start(c, CFD2D_K_STAGE);
+	switch (gr) {
+	case 1: hipLaunchKernelGGL((k_stage<MM, FLUX, VISC, 1>), g, blk, 0, c->st, a); break;
+	case 2: hipLaunchKernelGGL((k_stage<MM, FLUX, VISC, 2>), g, blk, 0, c->st, a); break;
+	case 3: hipLaunchKernelGGL((k_stage<MM, FLUX, VISC, 3>), g, blk, 0, c->st, a); break;
+	default: hipLaunchKernelGGL((k_stage<MM, FLUX, VISC, 4>), g, blk, 0, c->st, a); break;
+	}
+	rec_stop(c);
+}
+
+template <bool MM, bool VISC>
+void launch_stage_v(cfd2d_ctx* c, const Bufs& b, int mode, int nt)
+{
+	switch (c->p.flux) {
+	case CFD2D_FLUX_LAX: launch_stage_f<MM, CFD2D_FLUX_LAX, VISC>(c, b, mode, nt); break;
+	case CFD2D_FLUX_HLLC: launch_stage_f<MM, CFD2D_FLUX_HLLC, VISC>(c, b, mode, nt); break;
+	case CFD2D_FLUX_ROE: launch_stage_f<MM, CFD2D_FLUX_ROE, VISC>(c, b, mode, nt); break;
+	default:
+		if (c->ph.rk.gamma14) launch_stage_f<MM, FLUX_GODUNOV14, VISC>(c, b, mode, nt);
+		else launch_stage_f<MM, CFD2D_FLUX_GODUNOV, VISC>(c, b, mode, nt);
+		break;
+	}
+}
+
+// Stage s of a step: the stage kernel (fuse modes -1 and 2) or the gradient,
+// edge and update passes.  The stage kernel may not write the state it reads:
+// within a step it goes U -> U0 (-> U1) -> U (U, the step's start, is read by
+// its own cell alone in the later stages).  The stage kernel leaves the
+// primitives b.P behind (refresh_prim).
+template <bool MM>
+void launch_stage(cfd2d_ctx* c, int s)
+{
+	const int modes2[2] = {UPD_FIRST, UPD_RK2_LAST}, modes3[3] = {UPD_FIRST, UPD_RK3_MID, UPD_RK3_LAST};
+	int S = c->p.rk_stages, mode = S == 3 ? modes3[s] : modes2[s];
+	if (!stage_path(c)) {
+		launch_gradient_edge<MM>(c);
+		launch_update<MM>(c, mode);
+		return;
+	}
+	Bufs b = c->b;
+	double* at[3] = {c->b.U, c->b.U0, c->b.U1};
+	b.U = at[s];
+	b.U0 = c->b.U;
+	b.Un = s == S - 1 ? c->b.U : at[s + 1];
+	int nt = !c->ph.store_g && stream_state(c) ? 1 : 0;
+	if (c->p.viscous) launch_stage_v<MM, true>(c, b, mode, nt);
+	else launch_stage_v<MM, false>(c, b, mode, nt);
+}
+
 template <bool MM>
 void enqueue_step(cfd2d_ctx* c)
 {
-	if (c->p.steady) LAUNCH(c, CFD2D_K_TAU, (k_tau<MM>), c->nc, c->b, c->ph);
-	if (c->p.rk_stages == 3) {
-		const int modes[3] = {UPD_FIRST, UPD_RK3_MID, UPD_RK3_LAST};
-		for (int s = 0; s < 3; s++) {
-			launch_gradient_edge<MM>(c);
-			launch_update<MM>(c, modes[s]);
-		}
-	} else {
-		const int modes[2] = {UPD_FIRST, UPD_RK2_LAST};
-		for (int s = 0; s < 2; s++) {
-			launch_gradient_edge<MM>(c);
-			launch_update<MM>(c, modes[s]);
-		}
-	}
+	if (c->p.steady && !stage_path(c)) LAUNCH(c, CFD2D_K_TAU, (k_tau<MM>), c->nc, c->b, c->ph);
+	for (int s = 0; s < c->p.rk_stages; s++) launch_stage<MM>(c, s);
 	rec_start(c, CFD2D_K_REMEDIATE);
 	hipLaunchKernelGGL((k_remediate<MM>), dim3(1), dim3(BLOCK), 0, c->st, c->b, c->ph);
 	rec_stop(c);
@@ -1275,8 +1629,19 @@ void do_prim(cfd2d_ctx* c)
 	else launch_prim<false>(c);
 }
 
+// b.P is the state's: the stage kernel advances U alone, so whatever reads
+// b.P calls this first (never while a graph is being recorded: what is
+// recorded must not depend on it)
+void refresh_prim(cfd2d_ctx* c)
+{
+	if (!c->prim_stale) return;
+	do_prim(c);
+	c->prim_stale = false;
+}
+
 void do_gradient(cfd2d_ctx* c)
 {
+	refresh_prim(c);
 	if (c->mm) launch_gradient<true>(c);
 	else launch_gradient<false>(c);
 }
@@ -1287,6 +1652,15 @@ void do_edge(cfd2d_ctx* c)
 	else launch_edge<false>(c);
 }
 
+// the primitives' state around nsteps steps about to be enqueued: the passes
+// read and renew them, the stage kernel does neither
+void before_steps(cfd2d_ctx* c, int nsteps)
+{
+	if (nsteps <= 0) return;
+	if (!stage_path(c)) refresh_prim(c);
+	else c->prim_stale = true;
+}
+
 int check_launch(const char* what)
 {
 	hipError_t e = hipGetLastError();
@@ -1294,46 +1668,165 @@ int check_launch(const char* what)
 	return 0;
 }
 
-// least-squares weights w_k = A^{-1} d_k, A = sum d d^T (the oracle's lsq_weights)
-// Tiles of the tiled edge pass (k_edge_tile): tiles of T consecutive cells,
-// each owning the edges whose c1 it holds, staging c1 and (inner edges) c2
-// of those edges.  False when the edges are not in c1 order or a tile would
-// stage more than TILE_CAP cells.
-bool build_tiles(const std::vector<int>& c1, const std::vector<int>& c2, int nc, int T, std::vector<int>& tiles,
-                 std::vector<int>& tcell, std::vector<unsigned>& eslot)
+// Tiles of the stage pass (k_stage): the cells of each case in Hilbert order
+// of their centroids, cut greedily into tiles of at most `most` own cells
+// whose staged cells (own cells and those across their faces), all cells
+// (also those around the staged ones) and edges fit the shape's.  Within a
+// tile cells and edges ascend.
+struct Tiles {
+	std::vector<int4> head, rec, edge;  // edge: the edge, its lanes' cells (edge_pack's), whether to report
+	std::vector<int2> face;
+	std::vector<int> cell;
+	int all = 0, sc = 0, ec = 0;  // cells, staged cells and edges per tile in the arrays
+};
+
+void build_tiles(const Mesh& m, const std::vector<int>& c2, const std::vector<int>& cface,
+                 const std::vector<int>& cnb, bool limiter, int most, Tiles& out)
 {
-	int ne = (int)c1.size();
-	for (int e = 1; e < ne; e++)
-		if (c1[e] < c1[e - 1]) return false;
-	int nt = (nc + T - 1) / T;
-	tiles.assign(4 * (size_t)nt, 0);
-	tcell.clear();
-	eslot.assign(ne, 0u);
-	std::vector<int> need;
-	int e = 0;
-	for (int t = 0; t < nt; t++) {
-		int e0 = e;
-		while (e < ne && c1[e] < (t + 1) * T) e++;
-		need.clear();
-		for (int k = e0; k < e; k++) {
-			need.push_back(c1[k]);
-			if (c2[k] >= 0) need.push_back(c2[k]);
+	using Lim = StageShape<true>;
+	using Plain = StageShape<false>;
+	const int max_all = limiter ? Lim::ALL : Plain::ALL, max_staged = limiter ? Lim::CELLS : Plain::CELLS,
+	          max_edges = limiter ? Lim::EDGES : Plain::EDGES;
+	int nc = m.nc;
+	// Hilbert order, case by case (least-significant-digit radix sort of the keys)
+	std::vector<unsigned> key(nc), key2(nc);
+	std::vector<int> order(nc), order2(nc);
+	for (size_t k = 0; k + 1 < m.case_cell_offset.size(); k++) {
+		int a = m.case_cell_offset[k], z = m.case_cell_offset[k + 1];
+		if (z <= a) continue;
+		double lx = m.cx[a], hx = lx, ly = m.cy[a], hy = ly;
+		for (int i = a; i < z; i++) {
+			lx = std::min(lx, m.cx[i]);
+			hx = std::max(hx, m.cx[i]);
+			ly = std::min(ly, m.cy[i]);
+			hy = std::max(hy, m.cy[i]);
 		}
-		std::sort(need.begin(), need.end());
-		need.erase(std::unique(need.begin(), need.end()), need.end());
-		if ((int)need.size() > TILE_CAP) return false;
-		tiles[4 * (size_t)t] = (int)tcell.size();
-		tiles[4 * (size_t)t + 1] = (int)need.size();
-		tiles[4 * (size_t)t + 2] = e0;
-		tiles[4 * (size_t)t + 3] = e - e0;
-		auto slot = [&](int cell) { return (unsigned)(std::lower_bound(need.begin(), need.end(), cell) - need.begin()); };
-		for (int k = e0; k < e; k++) eslot[k] = slot(c1[k]) | ((c2[k] >= 0 ? slot(c2[k]) : 0xffffu) << 16);
-		tcell.insert(tcell.end(), need.begin(), need.end());
+		double sx = hx > lx ? 65535.0 / (hx - lx) : 0.0, sy = hy > ly ? 65535.0 / (hy - ly) : 0.0;
+		for (int i = a; i < z; i++) {
+			double qx = (m.cx[i] - lx) * sx, qy = (m.cy[i] - ly) * sy;  // a centroid that is no number sorts first
+			key[i] = (unsigned)hilbert_index(qx >= 0 ? std::min((int)qx, 65535) : 0,
+			                                 qy >= 0 ? std::min((int)qy, 65535) : 0, 16);
+			order[i] = i;
+		}
+		for (int shift = 0; shift < 32; shift += 11) {
+			unsigned count[2049] = {0};
+			for (int i = a; i < z; i++) count[((key[i] >> shift) & 2047u) + 1]++;
+			for (int d = 0; d < 2048; d++) count[d + 1] += count[d];
+			for (int i = a; i < z; i++) {
+				unsigned at = a + count[(key[i] >> shift) & 2047u]++;
+				key2[at] = key[i];
+				order2[at] = order[i];
+			}
+			std::copy(key2.begin() + a, key2.begin() + z, key.begin() + a);
+			std::copy(order2.begin() + a, order2.begin() + z, order.begin() + a);
+		}
 	}
-	if (tcell.empty()) tcell.push_back(0);
-	return e == ne;
+	// cut: per tile its cells (own, then those across their faces, then those
+	// around them) and edges, back to back.  cmark: 4 tile + 1 (own), 2 or 3
+	// of the last tile that holds the cell.
+	std::vector<int> cells, edges, start;  // start: 4 per tile, where its lists of cells and edges begin
+	std::vector<int> cmark(nc, 0), emark(m.ne, 0), cslot(nc, 0), eslot(m.ne, 0);
+	std::vector<int> own, ring, outer;
+	cells.reserve(nc + nc / 2);
+	edges.reserve(m.ne + m.ne / 4);
+	for (int at = 0, tile = 1; at < nc; tile++) {
+		own.clear();
+		ring.clear();
+		outer.clear();
+		int e0 = (int)edges.size(), staged = 0, all = 0, T = 4 * tile;
+		while (at < nc && (int)own.size() < most) {
+			// what cell i would add: itself and its neighbours to the staged
+			// cells, theirs to all cells, its edges
+			int i = order[at], add = cmark[i] > T && cmark[i] < T + 3 ? 0 : 1, eds = 0, far = 0;
+			if (cmark[i] <= T) far++;
+			for (int k = 0; k < 3; k++) {
+				int j = cnb[4 * (size_t)i + k];
+				if (emark[cface[4 * (size_t)i + k] >> 1] != tile) eds++;
+				if (j < 0) continue;
+				if (cmark[j] <= T || cmark[j] == T + 3) {
+					add++;
+					if (cmark[j] <= T) far++;
+					for (int q = 0; q < 3; q++) {
+						int x = cnb[4 * (size_t)j + q];
+						if (x >= 0 && cmark[x] <= T) far++;
+					}
+				}
+			}
+			if (staged + add > max_staged || all + far > max_all || (int)edges.size() - e0 + eds > max_edges) break;
+			auto enter = [&](int c, int as, std::vector<int>& list) {
+				if (cmark[c] <= T) all++;
+				if (as < 3 && (cmark[c] <= T || cmark[c] == T + 3)) staged++;
+				cmark[c] = T + as;
+				list.push_back(c);
+			};
+			enter(i, 1, own);
+			for (int k = 0; k < 3; k++) {
+				int j = cnb[4 * (size_t)i + k], e = cface[4 * (size_t)i + k] >> 1;
+				if (emark[e] != tile) {
+					emark[e] = tile;
+					edges.push_back(e);
+				}
+				if (j < 0 || (cmark[j] > T && cmark[j] != T + 3)) continue;
+				enter(j, 2, ring);
+				for (int q = 0; q < 3; q++) {
+					int x = cnb[4 * (size_t)j + q];
+					if (x >= 0 && cmark[x] <= T) enter(x, 3, outer);
+				}
+			}
+			at++;
+		}
+		// a cell listed further out may have moved in since
+		start.insert(start.end(), {(int)cells.size(), (int)own.size(), 0, e0});
+		std::vector<int>* lists[3] = {&own, &ring, &outer};
+		for (int r = 0; r < 3; r++) {
+			size_t c0 = cells.size();
+			for (int c : *lists[r])
+				if (cmark[c] == T + 1 + r) cells.push_back(c);
+			std::sort(cells.begin() + c0, cells.end());
+			if (r == 1) start[start.size() - 2] = (int)(cells.size() - start[start.size() - 4]);
+		}
+		std::sort(edges.begin() + e0, edges.end());
+		out.sc = std::max(out.sc, start[start.size() - 2]);
+		out.all = std::max(out.all, (int)cells.size() - start[start.size() - 4]);
+		out.ec = std::max(out.ec, (int)edges.size() - e0);
+	}
+	int nt = (int)(start.size() / 4);
+	start.insert(start.end(), {(int)cells.size(), 0, 0, (int)edges.size()});
+	out.all = (out.all + 15) / 16 * 16;
+	out.sc = (out.sc + 15) / 16 * 16;
+	out.ec = (out.ec + 15) / 16 * 16;
+	out.head.resize(nt);
+	out.cell.assign((size_t)nt * out.all, -1);
+	out.rec.assign((size_t)nt * out.sc, int4{-1, -1, -1, -1});
+	out.face.assign((size_t)nt * out.sc, int2{0, 0});
+	out.edge.assign((size_t)nt * out.ec, int4{-1, -1, -1, 0});
+	for (int tile = 0; tile < nt; tile++) {
+		const int* s = &start[4 * (size_t)tile];
+		const int *tc = &cells[s[0]], *te = &edges[s[3]];
+		int na = s[4] - s[0], no = s[1], ns = s[2], n = s[7] - s[3];
+		out.head[tile] = int4{no, ns, na, n};
+		std::copy(tc, tc + na, out.cell.begin() + (size_t)tile * out.all);
+		for (int k = 0; k < na; k++) cslot[tc[k]] = k;
+		for (int k = 0; k < n; k++) {
+			int e = te[k], c1 = m.c1[e];
+			eslot[e] = k;
+			bool mine = std::binary_search(tc, tc + no, c1);
+			out.edge[(size_t)tile * out.ec + k] = int4{e, cslot[c1], c2[e] >= 0 ? cslot[c2[e]] : c2[e], mine};
+		}
+		for (int k = 0; k < ns; k++) {
+			int i = tc[k], nj[3], f[3] = {0, 0, 0};
+			for (int q = 0; q < 3; q++) {
+				int fc = cface[4 * (size_t)i + q], j = cnb[4 * (size_t)i + q];
+				nj[q] = j >= 0 ? cslot[j] : -1 - (fc >> 1);
+				if (k < no) f[q] = 2 * eslot[fc >> 1] + (fc & 1);
+			}
+			out.rec[(size_t)tile * out.sc + k] = int4{nj[0], nj[1], nj[2], i};
+			out.face[(size_t)tile * out.sc + k] = int2{f[0] | f[1] << 16, f[2]};
+		}
+	}
 }
 
+// least-squares weights w_k = A^{-1} d_k, A = sum d d^T (the oracle's lsq_weights)
 void lsq_weights(const Mesh& m, std::vector<double>& w)
 {
 	int nc = m.nc;
@@ -1368,6 +1861,31 @@ void lsq_weights(const Mesh& m, std::vector<double>& w)
 			w[6 * (size_t)i + 2 * k + 1] = (a11 * d[k][1] - a12 * d[k][0]) / det;
 		}
 	}
+}
+
+// fills the tiles' static arrays on the device (null stream) from the edges'
+// midpoint offsets emid and signed lengths esl, held there for the call
+int fill_tiles(cfd2d_ctx* c, const std::vector<int4>& edges, const std::vector<double>& esl,
+               const std::vector<double>& emid)
+{
+	if (c->b.ntiles == 0) return 0;
+	size_t be = edges.size() * sizeof(int4), bs = (esl.size() + 1) / 2 * 16, bm = emid.size() * sizeof(double);
+	char* ws = nullptr;
+	HIPCHK(hipMalloc(&ws, be + bm + bs));
+	double* mid = (double*)(ws + be);
+	double* sl = (double*)(ws + be + bm);
+	hipError_t e = hipMemcpy(ws, edges.data(), be, hipMemcpyHostToDevice);
+	if (e == hipSuccess) e = hipMemcpy(mid, emid.data(), bm, hipMemcpyHostToDevice);
+	if (e == hipSuccess) e = hipMemcpy(sl, esl.data(), esl.size() * sizeof(double), hipMemcpyHostToDevice);
+	if (e == hipSuccess) {
+		hipLaunchKernelGGL(k_fill_tiles, dim3(c->b.ntiles), dim3(BLOCK), 0, 0, c->b,
+		                   (const double*)(c->b.lsqw ? c->b.lsqw : c->b.cfn), (const int4*)ws, (const double*)sl,
+		                   (const double*)mid);
+		e = hipGetLastError();
+	}
+	if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+	(void)hipFree(ws);
+	return e == hipSuccess ? 0 : hip_fail(e, "k_fill_tiles");
 }
 
 void drop_adj_graph(cfd2d_ctx::AdjGraph& a)
@@ -1472,6 +1990,7 @@ int cfd2d_ctx_create(const cfd2d_mesh* mesh, const cfd2d_params* p, int n_bc, co
 	c->case_tau.assign(c->ncase, p->tau);
 	c->hS = m.S;
 	c->hc1 = m.c1;
+	c->c1_order = std::is_sorted(m.c1.begin(), m.c1.end());
 	c->hel = m.l;
 	c->hnx = m.nx;
 	c->hny = m.ny;
@@ -1522,20 +2041,26 @@ int cfd2d_ctx_create(const cfd2d_mesh* mesh, const cfd2d_params* p, int n_bc, co
 		int cells[2] = {m.c1[e], ec2[e]};
 		memcpy(&eg[4 * (size_t)e + 3], cells, sizeof(cells));
 	}
-	std::vector<double> edl(8 * (size_t)ne, 0.0);
+	// Gauss-point offsets from the edge's midpoint (edge_offset); the second
+	// lane of a boundary edge reconstructs c1
+	std::vector<double> edl(8 * (size_t)ne, 0.0), esl(ne), emid(4 * (size_t)ne);
 	for (int e = 0; e < ne; e++) {
 		int c1 = m.c1[e], c2 = m.c2[e];
-		for (int g = 0; g < 2; g++) {
-			double px = m.gp[6 * (size_t)e + 2 + 2 * g], py = m.gp[6 * (size_t)e + 3 + 2 * g];
-			edl[edl_index(e, 0, g)] = px - m.cx[c1];
-			edl[edl_index(e, 0, g) + 1] = py - m.cy[c1];
-			if (c2 >= 0) {
-				edl[edl_index(e, 1, g)] = px - (m.cx[c2] + m.shx[e]);
-				edl[edl_index(e, 1, g) + 1] = py - (m.cy[c2] + m.shy[e]);
-			} else if (g == 1) {  // the second lane of a boundary edge reconstructs c1
-				edl[8 * (size_t)e + 4] = px - m.cx[c1];
-				edl[8 * (size_t)e + 5] = py - m.cy[c1];
+		const double* gp = &m.gp[6 * (size_t)e];
+		// whether the second Gauss point lies along (-ny, nx) from the first
+		bool along = (gp[5] - gp[3]) * m.nx[e] - (gp[4] - gp[2]) * m.ny[e] >= 0.0;
+		esl[e] = along ? m.l[e] : -m.l[e];
+		for (int side = 0; side < 2; side++) {
+			double mx = gp[0] - m.cx[c1], my = gp[1] - m.cy[c1];
+			if (side == 1 && c2 >= 0) {
+				mx = gp[0] - (m.cx[c2] + m.shx[e]);
+				my = gp[1] - (m.cy[c2] + m.shy[e]);
 			}
+			emid[4 * (size_t)e + 2 * side] = mx;
+			emid[4 * (size_t)e + 2 * side + 1] = my;
+			for (int g = 0; g < 2; g++)
+				if (side == 0 || c2 >= 0 || g == 1)
+					edge_offset(mx, my, m.nx[e], m.ny[e], esl[e], g, &edl[edl_index(e, side, g)]);
 		}
 	}
 	std::vector<double> bcp(4 * (size_t)(n_bc > 0 ? n_bc : 1), 0.0);
@@ -1562,24 +2087,21 @@ int cfd2d_ctx_create(const cfd2d_mesh* mesh, const cfd2d_params* p, int n_bc, co
 		return rc;
 	}
 	if (p->limiter != CFD2D_LIMITER_NONE) {
-		// each cell's offsets to the Gauss points of its faces, faces in
-		// ascending edge order (the limiter's order), from edl's own side
-		std::vector<double> cgp(12 * (size_t)nc);
+		// each cell's offsets to the midpoints of its first two faces (ascending
+		// edge order)
+		std::vector<double> cmid(4 * (size_t)nc);
 		for (int i = 0; i < nc; i++)
-			for (int k = 0; k < 3; k++) {
+			for (int k = 0; k < 2; k++) {
 				int f = cface[4 * (size_t)i + k];
-				int e = f >> 1, side = f & 1;
-				for (int g = 0; g < 2; g++) {
-					cgp[(size_t)(2 * (2 * k + g)) * nc + i] = edl[edl_index(e, side, g)];
-					cgp[(size_t)(2 * (2 * k + g) + 1) * nc + i] = edl[edl_index(e, side, g) + 1];
-				}
+				for (int q = 0; q < 2; q++)
+					cmid[(size_t)(2 * k + q) * nc + i] = emid[4 * (size_t)(f >> 1) + 2 * (f & 1) + q];
 			}
-		if ((rc = upload(c, &b.cgp, cgp))) {
+		if ((rc = upload(c, &b.cmid, cmid))) {
 			destroy_ctx(c);
 			return rc;
 		}
 	} else {
-		b.cgp = nullptr;
+		b.cmid = nullptr;
 	}
 	if (p->gradient == CFD2D_GRAD_LSQ) {
 		std::vector<double> w;
@@ -1591,21 +2113,27 @@ int cfd2d_ctx_create(const cfd2d_mesh* mesh, const cfd2d_params* p, int n_bc, co
 	} else {
 		b.lsqw = nullptr;
 	}
+	// measured on the periodic NS case: streaming loses 5 % with 272 MB of
+	// arrays (before the tiles'), gains 1.4 % with 544 MB and 2.5 % with 1.1 GB
+	c->stream_auto = c->dev_bytes > 2 * LLC_BYTES;
 	{
-		// the tiled edge pass: the largest tile whose staged set fits
-		std::vector<int> tiles, tcell;
-		std::vector<unsigned> eslot;
-		b.ntiles = 0;
-		for (int T : {TILE_CELLS, 192, 128, 96, 64})
-			if (build_tiles(m.c1, ec2, nc, T, tiles, tcell, eslot)) {
-				if ((rc = upload(c, &b.tiles, tiles)) || (rc = upload(c, &b.tcell, tcell)) ||
-				    (rc = upload(c, &b.eslot, eslot))) {
-					destroy_ctx(c);
-					return rc;
-				}
-				b.ntiles = (int)(tiles.size() / 4);
-				break;
-			}
+		Tiles t;
+		build_tiles(m, ec2, cface, cnb, p->limiter != CFD2D_LIMITER_NONE, tile_cells(nc), t);
+		size_t ns = t.rec.size(), es = t.edge.size();
+		b.ntiles = (int)t.head.size();
+		b.tall = t.all;
+		b.tsc = t.sc;
+		b.tec = t.ec;
+		b.tthreads = tile_threads(t.sc, t.ec);
+		b.tcmid = nullptr;
+		if ((p->rk_stages == 3 && (rc = dalloc(c, &b.U1, n4))) || (rc = upload(c, &b.thead, t.head)) ||
+		    (rc = upload(c, &b.tcell, t.cell)) || (rc = upload(c, &b.trec, t.rec)) ||
+		    (rc = upload(c, &b.tface, t.face)) || (rc = dalloc(c, &b.tw, 6 * ns)) ||
+		    (rc = dalloc(c, &b.tgeo, 4 * es)) || (rc = dalloc(c, &b.tmid, 4 * es)) ||
+		    (b.cmid && (rc = dalloc(c, &b.tcmid, 4 * ns))) || (rc = fill_tiles(c, t.edge, esl, emid))) {
+			destroy_ctx(c);
+			return rc;
+		}
 	}
 	hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
 	if (e != hipSuccess) {
@@ -1624,9 +2152,6 @@ int cfd2d_ctx_create(const cfd2d_mesh* mesh, const cfd2d_params* p, int n_bc, co
 		destroy_ctx(c);
 		return fail(CFD2D_ERR_HIP, "initial upload failed");
 	}
-	// measured on the periodic NS case: streaming loses 5 % with 272 MB of
-	// arrays, gains 1.4 % with 544 MB and 2.5 % with 1.1 GB
-	c->stream_auto = c->dev_bytes > 2 * LLC_BYTES;
 	*out = c;
 	return CFD2D_OK;
 }
@@ -1638,6 +2163,7 @@ int cfd2d_set_state(cfd2d_ctx* c, const double* u)
 	if (!c || !u) return fail(CFD2D_ERR_ARG, "null");
 	HIPCHK(hipMemcpyAsync(c->b.U, u, 4 * (size_t)c->nc * sizeof(double), hipMemcpyHostToDevice, c->st));
 	do_prim(c);
+	c->prim_stale = false;
 	HIPCHK(hipStreamSynchronize(c->st));
 	return check_launch("k_prim");
 }
@@ -1647,6 +2173,7 @@ int cfd2d_set_state_device(cfd2d_ctx* c, const double* du)
 	if (!c || !du) return fail(CFD2D_ERR_ARG, "null");
 	HIPCHK(hipMemcpyAsync(c->b.U, du, 4 * (size_t)c->nc * sizeof(double), hipMemcpyDeviceToDevice, c->st));
 	do_prim(c);
+	c->prim_stale = false;
 	HIPCHK(hipStreamSynchronize(c->st));
 	return check_launch("k_prim");
 }
@@ -1688,6 +2215,7 @@ int cfd2d_get_flags(cfd2d_ctx* c, unsigned* f)
 int cfd2d_calc_tau(cfd2d_ctx* c)
 {
 	if (!c) return fail(CFD2D_ERR_ARG, "null");
+	refresh_prim(c);
 	if (c->mm) LAUNCH(c, CFD2D_K_TAU, (k_tau<true>), c->nc, c->b, c->ph);
 	else LAUNCH(c, CFD2D_K_TAU, (k_tau<false>), c->nc, c->b, c->ph);
 	int rc = check_launch("k_tau");
@@ -1796,6 +2324,7 @@ int cfd2d_step(cfd2d_ctx* c, int nsteps)
 {
 	if (!c || nsteps < 0) return fail(CFD2D_ERR_ARG, "bad arguments");
 	if (c->prefer_graph && !c->timing) return cfd2d_step_graph(c, nsteps);
+	before_steps(c, nsteps);
 	for (int s = 0; s < nsteps; s++) step_once(c);
 	return check_launch("cfd2d_step");
 }
@@ -1809,6 +2338,7 @@ constexpr int GRAPH_STEPS = 500, GRAPH_KEEP = 4;
 int cfd2d_step_graph(cfd2d_ctx* c, int nsteps)
 {
 	if (!c || nsteps < 0) return fail(CFD2D_ERR_ARG, "bad arguments");
+	before_steps(c, nsteps);
 	while (nsteps > 0) {
 		int k = std::min(nsteps, GRAPH_STEPS);
 		hipGraphExec_t x = nullptr;
@@ -1867,6 +2397,7 @@ int cfd2d_wall_force(cfd2d_ctx* c, const int* mask, double* fx, double* fy)
 {
 	if (!c || !mask) return fail(CFD2D_ERR_ARG, "null");
 	std::vector<double> P(4 * (size_t)c->nc);
+	refresh_prim(c);
 	HIPCHK(hipStreamSynchronize(c->st));
 	HIPCHK(hipMemcpy(P.data(), c->b.P, P.size() * sizeof(double), hipMemcpyDeviceToHost));
 	double X = 0.0, Y = 0.0;
@@ -1905,8 +2436,8 @@ int cfd2d_stream_state(cfd2d_ctx* c, int mode)
 int cfd2d_fuse_gradient(cfd2d_ctx* c, int mode)
 {
 	if (!c || mode < -1 || mode > 2) return fail(CFD2D_ERR_ARG, "cfd2d_fuse_gradient: mode is -1, 0, 1 or 2");
-	if (mode == 2 && c->b.ntiles == 0)
-		return fail(CFD2D_ERR_ARG, "cfd2d_fuse_gradient: no tiled edge pass for this mesh (edges not in c1 order)");
+	if (mode == 2 && !c->c1_order)
+		return fail(CFD2D_ERR_ARG, "cfd2d_fuse_gradient: no tiled pass for this mesh (edges not in c1 order)");
 	c->fuse_mode = mode;
 	drop_graph(c);  // the recorded step holds the previous choice
 	return CFD2D_OK;
@@ -1930,6 +2461,7 @@ int cfd2d_autotune(cfd2d_ctx* c, int trial_steps, int* fuse_mode, int* use_graph
 		off[k] = total;
 		total += (parts[k].bytes + 255) & ~(size_t)255;
 	}
+	refresh_prim(c);  // saved and restored with the state
 	HIPCHK(hipStreamSynchronize(c->st));
 	char* save = nullptr;
 	HIPCHK(hipMalloc(&save, total));
@@ -1955,11 +2487,11 @@ int cfd2d_autotune(cfd2d_ctx* c, int trial_steps, int* fuse_mode, int* use_graph
 	int best_fuse = 0, best_graph = 0, best_stream = 0, best_shape = 0;
 	// the code-path variants with the default launch shape, then the launch
 	// shapes of the per-edge pass with the fastest of them
-	int nfuse = c->b.ntiles > 0 ? 3 : 2, nbase = 4 * nfuse;
+	const int nfuse = 3, nbase = 4 * nfuse;
 	for (int v = 0; v < nbase + EDGE_SHAPES - 1 && err == hipSuccess; v++) {
 		int fuse = v % nfuse, graph = (v / nfuse) & 1, strm = (v / nfuse / 2) & 1, shape = 0;
 		if (v >= nbase) {
-			if (best_fuse == 2) break;  // the tiled pass has one launch shape
+			if (best_fuse == 2) break;  // the stage pass has one launch shape
 			fuse = best_fuse;
 			graph = best_graph;
 			strm = best_stream;
@@ -1971,6 +2503,7 @@ int cfd2d_autotune(cfd2d_ctx* c, int trial_steps, int* fuse_mode, int* use_graph
 		c->edge_shape = shape;
 		drop_graph(c);
 		if ((err = copy_all(false)) != hipSuccess) break;
+		c->prim_stale = false;
 		if (cfd2d_step(c, graph ? trial_steps : 1) != CFD2D_OK) {  // warm-up (records the timed graph)
 			err = hipErrorUnknown;
 			break;
@@ -1993,6 +2526,7 @@ int cfd2d_autotune(cfd2d_ctx* c, int trial_steps, int* fuse_mode, int* use_graph
 		}
 	}
 	if (err == hipSuccess) err = copy_all(false);
+	if (err == hipSuccess) c->prim_stale = false;
 	if (err == hipSuccess) err = hipStreamSynchronize(c->st);
 	c->timing = timing;
 	drop_graph(c);
@@ -2004,6 +2538,7 @@ int cfd2d_autotune(cfd2d_ctx* c, int trial_steps, int* fuse_mode, int* use_graph
 		c->prefer_graph = graph0;
 		c->stream_mode = stream0;
 		c->edge_shape = shape0;
+		c->prim_stale = true;
 		return hip_fail(err, "cfd2d_autotune");
 	}
 	c->fuse_mode = best_fuse;

@@ -52,7 +52,7 @@ enum { CFD2D_NEWTON_CAP = 500 };  /* Newton iterations when cfd2d_params.max_new
 enum {
 	CFD2D_K_GRADIENT = 0, CFD2D_K_EDGE_FLUX = 1, CFD2D_K_UPDATE = 2, CFD2D_K_REMEDIATE = 3,
 	CFD2D_K_TAU = 4, CFD2D_K_PRIM = 5, CFD2D_K_IMPL_GRADIENT = 6, CFD2D_K_IMPL_EDGE = 7,
-	CFD2D_K_IMPL_ASSEMBLE = 8, CFD2D_K_COUNT = 9
+	CFD2D_K_IMPL_ASSEMBLE = 8, CFD2D_K_STAGE = 9, CFD2D_K_COUNT = 10
 };
 
 /*
@@ -171,17 +171,17 @@ int  cfd2d_status(cfd2d_ctx* c, long long* newton_cap_hits, int* nonfinite);
 int  cfd2d_wall_force(cfd2d_ctx* c, const int* edge_mask, double* fx, double* fy);
 /* per-kernel HIP-event timing on the context stream */
 int  cfd2d_timing(cfd2d_ctx* c, int enable);
-/* Where the cell gradients are formed: mode 1 in the edge pass itself (each
- * edge's lane pair forms its two cells'), 2 in the tiled edge pass (a
- * workgroup per tile of consecutive cells forms the gradients its edges
- * read once each, staged in LDS; CFD2D_ERR_ARG when the mesh's edges are
- * not in c1 order), 0 in a separate gradient pass whose records the edge
- * pass reads, -1 (default) 1 without a limiter and 0 with one.  All modes
- * give the same bits.  No reference counterpart. */
+/* How a stage is split into kernels: mode 2 or -1 (the default) one kernel by
+ * tiles of neighbouring cells, which keeps primitives, gradients and fluxes in
+ * LDS (2 returns CFD2D_ERR_ARG when the mesh's edges are not in c1 order);
+ * 1 an edge pass that forms the gradients itself (each edge's lane pair its
+ * two cells') and an update pass; 0 a separate gradient pass, an edge pass
+ * that reads its records and an update pass.  All modes give the same bits.
+ * No reference counterpart. */
 int  cfd2d_fuse_gradient(cfd2d_ctx* c, int mode);
 /* Whether the update pass reads and writes the conserved state with
  * non-temporal loads and stores (kept out of the caches, leaving them to the
- * data the edge pass gathers): 1 yes, 0 no, -1 (default) when the context's
+ * data that neighbours gather): 1 yes, 0 no, -1 (default) when the context's
  * device arrays are over twice the 256 MB Infinity Cache.  The same bits
  * either way.  No reference counterpart. */
 int  cfd2d_stream_state(cfd2d_ctx* c, int mode);
@@ -192,9 +192,9 @@ int  cfd2d_stream_state(cfd2d_ctx* c, int mode);
  * single-material contexts' unlimited and stored-gradient edge passes. */
 int  cfd2d_edge_shape(cfd2d_ctx* c, int shape);
 /* Autotuner (no reference counterpart): times trial_steps steps of each
- * variant -- gradients in their own pass, in the edge pass or in the tiled
- * edge pass (when the mesh has tiles), eager launches
- * or a replayed recorded step, cached or streamed state in the update pass
+ * variant -- a stage as three passes, two passes or one kernel
+ * (cfd2d_fuse_gradient), eager launches
+ * or a replayed recorded step, cached or streamed state in the update
  * -- on the context's current state, then the edge pass's launch shapes
  * (cfd2d_edge_shape) with the fastest of them, restores that state exactly,
  * and keeps the fastest for cfd2d_step (same results either way).  Reports
