@@ -18,13 +18,14 @@
 // of the ghost on boundaries and of the reconstruction into (P, G) adjoints
 // per cell: for HLLC and the exact Godunov flux (VJPs heavy in VALU
 // work) once per edge, k_adj_edge (two lanes
-// per edge, one Gauss point each, into a per-edge buffer for both sides) then
-// k_adj_cell (each cell gathers its faces' entries in ascending edge order);
-// for LAX k_adj_face (each cell evaluates its three faces from its own side,
-// no edge buffer; with geometry terms k_adj_edge's geometry-only mode beside
-// it).  Then k_adj_grad: reverse of the gradient operator (own
-// and neighbours' gradient adjoints, ghost terms), the primitive->conserved
-// Jacobian and the RK bookkeeping.  Boundary-parameter
+// per edge, one Gauss point each, into a per-edge buffer for both sides), which
+// each cell gathers from its faces' entries in ascending edge order; for LAX
+// k_adj_face (each cell evaluates its three faces from its own side, no edge
+// buffer; with geometry terms k_adj_edge's geometry-only mode beside it).  Then
+// the reverse of the gradient operator (own and neighbours' gradient adjoints,
+// ghost terms), the primitive->conserved Jacobian and the RK bookkeeping: with
+// the gather in one kernel by tiles, k_adj_tile, for HLLC and Godunov without
+// geometry terms, else k_adj_grad behind k_adj_face or k_adj_cell.  Boundary-parameter
 // adjoints accumulate per boundary edge and are summed per boundary object
 // once, in an order fixed by the launch shape.  No floating-point atomics:
 // the result does not depend on scheduling.
@@ -39,15 +40,19 @@
 
 namespace {
 
-constexpr int EA = 16;  // per edge [side][Gauss point][r, p, u, v]; on a boundary the
-                        // c2 half holds the adjoint of the ghost's cell-centre input
+// per edge [Gauss point][side][r, p, u, v], a record of 128 bytes: what a lane
+// of k_adj_edge writes is 64 bytes in a row, what one of the cell's pair reads
+// 32 of them, in whatever order its cells' edges are numbered (component arrays
+// cost a 64-byte sector per value where they are not the cells' own); on a
+// boundary side 1 holds the adjoint of the ghost's cell-centre input
+constexpr int EA = 16;
 
 struct AdjBufs {
 	double* Wn;     // [nc][4] dJ/dU_{s+1}
 	double* Ws;     // [nc][4] dJ/dU_s
 	double* Acc;    // [nc][4] sum of a * W over the stages of the current step
-	double* Pb;     // [4][nc] adjoint of the primitives
-	double* Gb;     // [8][nc] adjoint of the gradients
+	double* Pb;     // [4][nc] adjoint of the primitives, and
+	double* Gb;     // [8][nc] of the gradients, unless k_adj_tile holds them
 	                // (component arrays: held as per-cell records, the gfx950
 	                // build of k_adj_grad returned wrong boundary-cell values
 	                // at -O2/-O3, correct at -O1 or -fno-unroll-loops; both
@@ -55,7 +60,7 @@ struct AdjBufs {
 	                // UBSan with bounds checks and agree bitwise, so the source
 	                // holds no out-of-bounds or uninitialised access that would
 	                // explain it -- tests/test_hostemu.py)
-	double* Ea;     // [16][ne]
+	double* Ea;     // [ne][16]
 	double* Ebc;    // [8][ne] boundary-parameter adjoints per edge, summed over stages
 	                // (two slots of 4: one per Gauss point of the edge pass)
 	double* bcbar;  // [nbc][4]
@@ -150,8 +155,8 @@ __device__ __forceinline__ void lax_vjp(const Prim& L, const Prim& R, double nx,
                                         double* fo = nullptr)
 {
 	double unl = L.u * nx + L.v * ny, unr = R.u * nx + R.v * ny;
-	double irl = 1.0 / L.r, irr = 1.0 / R.r;
-	double cl = sqrt(G * L.p * irl), cr = sqrt(G * R.p * irr);
+	double irl = rcp_dev(L.r), irr = rcp_dev(R.r);
+	double cl = sqrt_dev(G * L.p * irl), cr = sqrt_dev(G * R.p * irr);
 	double al = fabs(unl) + cl, ar = fabs(unr) + cr;
 	bool left = al > ar;
 	double alpha = left ? al : ar;
@@ -173,7 +178,7 @@ __device__ __forceinline__ void lax_vjp(const Prim& L, const Prim& R, double nx,
 	// alpha = |u.n| + c of the side with the larger value
 	double cs = left ? cl : cr, ps = left ? L.p : R.p, irs = left ? irl : irr;
 	double ts = alb * 0.5 * cs;
-	double psb = ts / ps, rsb = -ts * irs;
+	double psb = ts * rcp_dev(ps), rsb = -ts * irs;
 	if (left) {
 		unlb += alb * (unl < 0 ? -1.0 : 1.0);
 		Lpb += psb;
@@ -217,8 +222,8 @@ __device__ __forceinline__ void lax_vjp_own(const Prim& L, const Prim& R, double
                                             double igm1, const double* fb, bool own_c2, double* Lb)
 {
 	double unl = L.u * nx + L.v * ny, unr = R.u * nx + R.v * ny;
-	double irl = 1.0 / L.r, irr = 1.0 / R.r;
-	double cl = sqrt(G * L.p * irl), cr = sqrt(G * R.p * irr);
+	double irl = rcp_dev(L.r), irr = rcp_dev(R.r);
+	double cl = sqrt_dev(G * L.p * irl), cr = sqrt_dev(G * R.p * irr);
 	double al = fabs(unl) + cl, ar = fabs(unr) + cr;
 	bool own = own_c2 ? !(ar > al) : al > ar;  // the forward pass's al > ar, seen from this side
 	double alpha = own ? al : ar;
@@ -235,7 +240,7 @@ __device__ __forceinline__ void lax_vjp_own(const Prim& L, const Prim& R, double
 	if (own) {
 		double ts = alb * 0.5 * cl;
 		unlb += alb * (unl < 0 ? -1.0 : 1.0);
-		Lpb += ts / L.p;
+		Lpb += ts * rcp_dev(L.p);
 		Lrb += -ts * irl;
 	}
 	Lrb += rolb + rulb * L.u + rvlb * L.v + relb * kl;
@@ -936,18 +941,18 @@ __device__ __forceinline__ void euler_flux_rev(const Prim& W, double un, double 
 }
 
 // the state's own terms: E = p/(G - 1) + r |u|^2 / 2, c = sqrt(G p / r),
-// un = u nx + v ny
-__device__ __forceinline__ void side_rev(const Prim& W, double c, double nx, double ny, double G, SideAdj& a,
-                                         double* Wb, double& nxb, double& nyb)
+// un = u nx + v ny (ir = 1/r, igm1 = 1/(G - 1))
+__device__ __forceinline__ void side_rev(const Prim& W, double ir, double c, double nx, double ny, double G,
+                                         double igm1, SideAdj& a, double* Wb, double& nxb, double& nyb)
 {
 	double r = a.r, p = a.p, u = a.u, v = a.v;
-	p += a.E / (G - 1.0);
+	p += a.E * igm1;
 	r += a.E * 0.5 * (W.u * W.u + W.v * W.v);
 	u += a.E * W.r * W.u;
 	v += a.E * W.r * W.v;
-	double ab = a.c / (2.0 * c);  // c = sqrt(a), a = G p / r
-	p += ab * G / W.r;
-	r -= ab * (G * W.p) / (W.r * W.r);
+	double ab = a.c * 0.5 * rcp_dev(c) * G * ir;  // c = sqrt(a), a = G p / r
+	p += ab;
+	r -= ab * W.p * ir;
 	u += a.un * nx;
 	v += a.un * ny;
 	nxb += a.un * W.u;
@@ -961,13 +966,14 @@ __device__ __forceinline__ void side_rev(const Prim& W, double c, double nx, dou
 // The HLLC flux's vector-Jacobian product (flux_hllc reversed by hand: the
 // outer states' Euler fluxes, or the contact speed, star state and wave
 // speeds of the star region); nb (if given) takes the normal's adjoint
-__device__ __forceinline__ void hllc_vjp(const Prim& L, const Prim& R, double nx, double ny, double G, const double* fb,
-                                         double* Lb, double* Rb, double* nb = nullptr, double* fo = nullptr)
+__device__ __forceinline__ void hllc_vjp(const Prim& L, const Prim& R, double nx, double ny, double G, double igm1,
+                                         const double* fb, double* Lb, double* Rb, double* nb = nullptr, double* fo = nullptr)
 {
 	double unl = L.u * nx + L.v * ny, unr = R.u * nx + R.v * ny;
-	double cl = sqrt(G * L.p / L.r), cr = sqrt(G * R.p / R.r);
-	double El = L.p / (G - 1.0) + 0.5 * L.r * (L.u * L.u + L.v * L.v);
-	double Er = R.p / (G - 1.0) + 0.5 * R.r * (R.u * R.u + R.v * R.v);
+	double irl = rcp_dev(L.r), irr = rcp_dev(R.r);
+	double cl = sqrt_dev(G * L.p * irl), cr = sqrt_dev(G * R.p * irr);
+	double El = L.p * igm1 + 0.5 * L.r * (L.u * L.u + L.v * L.v);
+	double Er = R.p * igm1 + 0.5 * R.r * (R.u * R.u + R.v * R.v);
 	double a1 = unl - cl, a2 = unr - cr, b1 = unl + cl, b2 = unr + cr;
 	bool sl1 = a1 < a2, sr1 = b1 > b2;
 	double sl = sl1 ? a1 : a2, sr = sr1 ? b1 : b2;
@@ -985,15 +991,15 @@ __device__ __forceinline__ void hllc_vjp(const Prim& L, const Prim& R, double nx
 		}
 	} else {
 		double ml = L.r * (sl - unl), mr = R.r * (sr - unr);
-		double num = R.p - L.p + L.r * unl * (sl - unl) - R.r * unr * (sr - unr), dens = ml - mr;
-		double ss = num / dens;
+		double num = R.p - L.p + L.r * unl * (sl - unl) - R.r * unr * (sr - unr), ids = rcp_dev(ml - mr);
+		double ss = num * ids;
 		bool lft = ss >= 0.0;
 		const Prim& K = lft ? L : R;
 		SideAdj& ak = lft ? al : ar;
-		double sk = lft ? sl : sr, unk = lft ? unl : unr, Ek = lft ? El : Er, mk = lft ? ml : mr;
-		double g = sk - ss, k = mk / g;
-		double d = ss - unk, e = sk - unk, he = K.r * e, h = K.p / he;
-		double B3 = ss + h, inner = Ek / K.r + d * B3;
+		double sk = lft ? sl : sr, unk = lft ? unl : unr, Ek = lft ? El : Er, mk = lft ? ml : mr, irk = lft ? irl : irr;
+		double ig = rcp_dev(sk - ss), k = mk * ig;
+		double d = ss - unk, e = sk - unk, ihe = rcp_dev(K.r * e), h = K.p * ihe;
+		double B3 = ss + h, inner = Ek * irk + d * B3;
 		double us1 = k * (K.u + d * nx), us2 = k * (K.v + d * ny), us3 = k * inner;
 		if (fo) {
 			fo[0] = K.r * unk + sk * (k - K.r);
@@ -1011,12 +1017,12 @@ __device__ __forceinline__ void hllc_vjp(const Prim& L, const Prim& R, double nx
 		euler_flux_rev(K, unk, Ek, nx, ny, fb, ak, nxb, nyb);
 		// us3 = k (Ek/Kr + d (ss + Kp / (Kr e)))
 		double kb = us3b * inner, innerb = us3b * k;
-		ak.E += innerb / K.r;
-		ak.r -= innerb * Ek / (K.r * K.r);
+		ak.E += innerb * irk;
+		ak.r -= innerb * Ek * irk * irk;
 		double db = innerb * B3, B3b = innerb * d;
 		double ssb = B3b, hb = B3b;
-		ak.p += hb / he;
-		double heb = -hb * K.p / (he * he);
+		ak.p += hb * ihe;
+		double heb = -hb * h * ihe;
 		ak.r += heb * e;
 		double eb = heb * K.r;
 		skb += eb;
@@ -1031,11 +1037,11 @@ __device__ __forceinline__ void hllc_vjp(const Prim& L, const Prim& R, double nx
 		ssb += db;
 		ak.un -= db;
 		// k = mk / (sk - ss)
-		double mkb = kb / g, gb = -kb * mk / (g * g);
+		double mkb = kb * ig, gb = -kb * k * ig;
 		skb += gb;
 		ssb -= gb;
 		// ss = (Rp - Lp + Lr unl (sl - unl) - Rr unr (sr - unr)) / (ml - mr)
-		double numb = ssb / dens, densb = -ssb * num / (dens * dens);
+		double numb = ssb * ids, densb = -ssb * ss * ids;
 		double mlb = densb + (lft ? mkb : 0.0), mrb = -densb + (lft ? 0.0 : mkb);
 		ar.p += numb;
 		al.p -= numb;
@@ -1053,8 +1059,8 @@ __device__ __forceinline__ void hllc_vjp(const Prim& L, const Prim& R, double nx
 		at.un += srb;
 		at.c += srb;
 	}
-	side_rev(L, cl, nx, ny, G, al, Lb, nxb, nyb);
-	side_rev(R, cr, nx, ny, G, ar, Rb, nxb, nyb);
+	side_rev(L, irl, cl, nx, ny, G, igm1, al, Lb, nxb, nyb);
+	side_rev(R, irr, cr, nx, ny, G, igm1, ar, Rb, nxb, nyb);
 	if (nb) {
 		nb[0] = nxb;
 		nb[1] = nyb;
@@ -1102,7 +1108,7 @@ __global__ __launch_bounds__(BLOCK) void k_adj_edge(Bufs b, Phys ph, AdjBufs a, 
 	}
 	double Lb[4], Rb[4], nb[2] = {0.0, 0.0};
 	double Fe[4];  // GEO: the stage's flux through the edge, from the VJP's own evaluation
-	if (FLUX == CFD2D_FLUX_HLLC) hllc_vjp(L, R, nx, ny, ph.gam_flux, fb, Lb, Rb, GEO ? nb : nullptr, GEO ? Fe : nullptr);
+	if (FLUX == CFD2D_FLUX_HLLC) hllc_vjp(L, R, nx, ny, ph.gam_flux, ph.igm1, fb, Lb, Rb, GEO ? nb : nullptr, GEO ? Fe : nullptr);
 	else if (FLUX == CFD2D_FLUX_GODUNOV)
 		godunov_vjp(L, R, nx, ny, ph.rk, ph.max_newton, fb, Lb, Rb, GEO ? nb : nullptr, GEO ? Fe : nullptr);
 	else lax_vjp(L, R, nx, ny, ph.gam_flux, ph.igm1, fb, Lb, Rb, GEO ? nb : nullptr, GEO ? Fe : nullptr);
@@ -1125,11 +1131,10 @@ __global__ __launch_bounds__(BLOCK) void k_adj_edge(Bufs b, Phys ph, AdjBufs a, 
 	} else {
 		for (int q = 0; q < 4; q++) Rsb[q] = Rb[q];
 	}
-	if (!GONLY)
-		for (int q = 0; q < 4; q++) {
-			a.Ea[(size_t)(4 * gp + q) * ne + e] = Lb[q];
-			a.Ea[(size_t)(8 + 4 * gp + q) * ne + e] = Rb[q];
-		}
+	if (!GONLY) {
+		st4(a.Ea, 4 * (size_t)e + 2 * gp, Lb);
+		st4(a.Ea, 4 * (size_t)e + 2 * gp + 1, Rb);
+	}
 	if (GEO) {
 		// this lane's Gauss point: the normal, and each side's offset (the
 		// reconstruction phi + g . d gives d-bar = sum_q phi-bar_q g_q)
@@ -1273,35 +1278,48 @@ __global__ __launch_bounds__(BLOCK) void k_adj_face(Bufs b, Phys ph, AdjBufs a, 
 	}
 }
 
-// each cell gathers its side of its three edges: P adjoint = sum of the
-// Gauss-point adjoints, G adjoint = sum of adjoint x Gauss-point offset
+// a cell's (P, G) adjoints from its faces' edge entries by its lane pair, one
+// Gauss point each: P adjoint = sum of the entries (on a boundary of the ghost's
+// cell-centre input too), G adjoint = sum of the entries times the offsets
+__device__ __forceinline__ void gather_edge_adj(const Bufs& b, const AdjBufs& a, const int* fs, const int* nj, int gp,
+                                                double* pb, double* gb)
+{
+#pragma unroll
+	for (int k = 0; k < 3; k++) {
+		int e = fs[k] >> 1, side = fs[k] & 1;
+		double dx = b.edl[edl_index(e, side, gp)], dy = b.edl[edl_index(e, side, gp) + 1];
+		double v[4];
+		ld4(a.Ea, 4 * (size_t)e + 2 * gp + side, v);
+		for (int q = 0; q < 4; q++) {
+			pb[q] += v[q];
+			gb[2 * q] += v[q] * dx;
+			gb[2 * q + 1] += v[q] * dy;
+		}
+		if (nj[k] < 0) {
+			ld4(a.Ea, 4 * (size_t)e + 2 * gp + 1, v);
+			for (int q = 0; q < 4; q++) pb[q] += v[q];
+		}
+	}
+	for (int q = 0; q < 4; q++) pb[q] += pair_swap(pb[q]);
+	for (int q = 0; q < 8; q++) gb[q] += pair_swap(gb[q]);
+}
+
+// Each cell gathers its side of its three edges (HLLC and Godunov with geometry
+// terms; without them k_adj_tile).  Two lanes per cell, one Gauss point each
 __global__ __launch_bounds__(BLOCK) void k_adj_cell(Bufs b, AdjBufs a)
 {
-	int i = xcd_block() * BLOCK + threadIdx.x;
-	if (i >= b.nc) return;
-	size_t ne = b.ne;
+	int t = xcd_block() * BLOCK + threadIdx.x;
+	int i = t >> 1, gp = t & 1;
+	if (i >= b.nc) return;  // both lanes of a pair leave together
 	double pb[4] = {0, 0, 0, 0};
 	double gb[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-	CellTop tp = load_top(b, i);
-	for (int k = 0; k < 3; k++) {
-		int f = tp.f[k];
-		int e = f >> 1, side = f & 1;
-		for (int gp = 0; gp < 2; gp++) {
-			double dx = b.edl[edl_index(e, side, gp)];
-			double dy = b.edl[edl_index(e, side, gp) + 1];
-			for (int q = 0; q < 4; q++) {
-				double v = a.Ea[(size_t)(8 * side + 4 * gp + q) * ne + e];
-				pb[q] += v;
-				gb[2 * q] += v * dx;
-				gb[2 * q + 1] += v * dy;
-			}
-		}
-		if (tp.nb[k] < 0)
-			for (int gp = 0; gp < 2; gp++)
-				for (int q = 0; q < 4; q++) pb[q] += a.Ea[(size_t)(8 + 4 * gp + q) * ne + e];
+	int4 fc = load_faces(b, i), nb = reinterpret_cast<const int4*>(b.cnb)[i];
+	int fs[3] = {fc.x, fc.y, fc.z}, nj[3] = {nb.x, nb.y, nb.z};
+	gather_edge_adj(b, a, fs, nj, gp, pb, gb);
+	if (gp == 0) {
+		sta4(a.Pb, b.nc, i, pb);
+		sta8(a.Gb, b.nc, i, gb);
 	}
-	sta4(a.Pb, b.nc, i, pb);
-	sta8(a.Gb, b.nc, i, gb);
 }
 
 // Reverse of the gradient operator and of the primitive conversion, then the
@@ -1437,6 +1455,163 @@ __global__ __launch_bounds__(BLOCK) void k_adj_grad(Bufs b, Phys ph, AdjBufs a, 
 	if (MODE != 2) store_records<4>(a.Acc, c0, nv, acc, lds_a);
 }
 
+// Own half of the gradient operator's reverse: from a cell's gradient adjoint
+// gb and weight record w, per face k the adjoint nbb[k] of the neighbour value
+// that it took, the cell's own part added to pb; half: the two components of
+// nbb that this lane of the cell's pair passes on.
+template <bool LSQ>
+__device__ __forceinline__ void own_gradient_adj(const double* w, double S, int gp, const double* gb, double* pb,
+                                                 double (*nbb)[4], double (*half)[2])
+{
+	double h = LSQ ? 1.0 : 0.5 * rcp_dev(S);
+#pragma unroll
+	for (int k = 0; k < 3; k++) {
+		// least squares takes w_k (phi_k - phi_i), Green-Gauss n l (phi_i + phi_k) / 2 / S
+		double wx = w[2 * k] * h, wy = w[2 * k + 1] * h;
+		double v0 = wx * gb[0] + wy * gb[1], v1 = wx * gb[2] + wy * gb[3];
+		double v2 = wx * gb[4] + wy * gb[5], v3 = wx * gb[6] + wy * gb[7];
+		const double sg = LSQ ? -1.0 : 1.0;
+		pb[0] += sg * v0;
+		pb[1] += sg * v1;
+		pb[2] += sg * v2;
+		pb[3] += sg * v3;
+		nbb[k][0] = v0;
+		nbb[k][1] = v1;
+		nbb[k][2] = v2;
+		nbb[k][3] = v3;
+		half[k][0] = gp ? v2 : v0;
+		half[k][1] = gp ? v3 : v1;
+	}
+}
+
+// a boundary face's nbb taken back through the ghost of the cell-centre state;
+// one lane of the pair (store) adds the parameters' adjoints
+__device__ __forceinline__ void ghost_gradient_adj(const Bufs& b, const AdjBufs& a, int e, bool store, const Prim& pi,
+                                                   const MatV& m, const double* nbb, double* pb)
+{
+	size_t ne = b.ne;
+	int bc = -edge_cells(b, e).y - 1;
+	double dL[4], dC[4], dpar[4];
+	ghost_vjp(b.bctype[bc], &b.bcpar[4 * bc], edge_geo(b, e)[0], edge_geo(b, e)[1], pi, pi, m, nbb, dL, dC, dpar,
+	          nullptr);
+	for (int q = 0; q < 4; q++) {
+		pb[q] += dL[q] + dC[q];
+		if (store) a.Ebc[(size_t)q * ne + e] += dpar[q];
+	}
+}
+
+// The end of a cell's reverse by its lane pair: the neighbours' gradients' part
+// o (this lane's components) joins pb, then P = (r, p, u, v)(U) transposed and
+// the RK bookkeeping, Ws = b W + (dP/dU)^T Pb and acc0 per MODE (0: Acc = a W,
+// 1: Acc += a W, 2: Ws += Acc, the step's first stage), two rows per lane.
+template <int MODE>
+__device__ __forceinline__ void adj_finish(const AdjBufs& a, int i, int gp, bool store, const Prim& pi, const MatV& m,
+                                           const double* o, double* pb, double wa, double wb)
+{
+	double o0 = o[0], o1 = o[1], x0 = pair_swap(o0), x1 = pair_swap(o1);
+	pb[0] += gp ? x0 : o0;
+	pb[1] += gp ? x1 : o1;
+	pb[2] += gp ? o0 : x0;
+	pb[3] += gp ? o1 : x1;
+	if (!store) return;
+	double ir = rcp_dev(pi.r), u = pi.u, v = pi.v, g1 = m.gam - 1.0;
+	double ub[2];
+	if (gp == 0) {
+		ub[0] = pb[0] - (pb[2] * u + pb[3] * v) * ir + pb[1] * g1 * 0.5 * (u * u + v * v);
+		ub[1] = pb[2] * ir - pb[1] * g1 * u;
+	} else {
+		ub[0] = pb[3] * ir - pb[1] * g1 * v;
+		ub[1] = pb[1] * g1;
+	}
+	size_t at = 4 * (size_t)i + 2 * gp;
+	const double* wn = static_cast<const double*>(__builtin_assume_aligned(a.Wn + at, 16));
+	double* wo = static_cast<double*>(__builtin_assume_aligned(a.Ws + at, 16));
+	double* ac = static_cast<double*>(__builtin_assume_aligned(a.Acc + at, 16));
+	for (int q = 0; q < 2; q++) {
+		double w = wn[q], ws = wb * w + ub[q];
+		if (MODE == 0) ac[q] = wa * w;
+		else if (MODE == 1) ac[q] += wa * w;
+		else ws += ac[q];
+		wo[q] = ws;
+	}
+}
+
+// whether a lane runs a part of a kernel that holds lane exchanges: the lanes
+// it concerns on the device; every lane where a workgroup's threads meet at
+// each exchange (a host build), the others on a cell of their own choice
+__device__ __forceinline__ bool takes_part(bool live)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+	return live;
+#else
+	(void)live;
+	return true;
+#endif
+}
+
+// The rest of a stage's reverse behind k_adj_edge (no geometry terms), by the
+// stage kernel's tiles: k_adj_cell and k_adj_grad in one.  Two lanes per
+// staged cell, one Gauss point each, gather the cell's (P, G) adjoints from
+// the edge entries and form from them, per face, the adjoint nbb of the
+// neighbour value that the cell's gradient took; these go to LDS, each own
+// cell adds its neighbours', and the pair finishes the cell (adj_finish).  The
+// (P, G) adjoints, 96 bytes per cell written, read and gathered from three
+// neighbours, never reach memory; a cell next to another tile is formed by
+// both.  Bound by its loads' latency where tiles are few, by the edge entries'
+// bytes where they are many.  Per stage 8.8 + 11.0 -> 12.5 us at 75 k cells
+// (Green-Gauss), 4.5 + 8.0 -> 7.5 at 8 k (least squares); a whole HLLC adjoint
+// of 501 k cells 8.98 -> 8.63 ms, of 864 cells 1.15 -> 0.95.  With the edge
+// entries as component arrays 15.4 and 10.1: a tile's edges are not in a row.
+// (LAX keeps k_adj_face and k_adj_grad: its VJPs from LDS in the same way took
+// 148 us per stage of 501 k cells at 164 registers and 190 held to 128, against
+// 64 + 31; k_adj_face handing on nbb records instead of (P, G) adjoints 79 + 32.)
+constexpr int ADJ_THREADS = (2 * StageShape<false>::CELLS + 63) / 64 * 64;
+
+template <bool MM, bool LSQ, int MODE>
+__global__ __attribute__((amdgpu_flat_work_group_size(1, ADJ_THREADS), amdgpu_waves_per_eu(4))) void k_adj_tile(
+    Bufs b, Phys ph, AdjBufs a, double wa, double wb)
+{
+	// nbb of the staged cells' faces k: (r, p) at 2 k, (u, v) at 2 k + 1
+	__shared__ __align__(16) double nb[6][StageShape<false>::CELLS][2];
+	int tile = xcd_block(), t = threadIdx.x, gp = t & 1;
+	int4 hd = b.thead[tile];
+	size_t n = b.nc, cb = (size_t)tile * b.tsc;
+	int slot = min(t >> 1, hd.y - 1);
+	bool staged = (t >> 1) < hd.y, own = (t >> 1) < hd.x;
+	int4 rc = b.trec[cb + slot];
+	int i = rc.w, nj[3] = {rc.x, rc.y, rc.z};
+	Prim pi{};
+	double pb[4] = {0, 0, 0, 0}, nbb[3][4];
+	if (takes_part(staged)) {
+		double gb[8] = {0, 0, 0, 0, 0, 0, 0, 0}, w[6], half[3][2];
+		int4 fc = load_faces(b, i);
+		int fs[3] = {fc.x, fc.y, fc.z};
+		pi = load_prim(b, i);
+		gather_edge_adj(b, a, fs, nj, gp, pb, gb);
+		ld6(b.tw + 6 * (cb + slot), w);
+		own_gradient_adj<LSQ>(w, LSQ ? 0.0 : b.S[i], gp, gb, pb, nbb, half);
+		if (staged)
+			for (int k = 0; k < 3; k++) st2(nb[2 * k + gp], slot, half[k]);
+	}
+	__syncthreads();
+	if (takes_part(own)) {
+		double o[2] = {0.0, 0.0};  // the neighbours' gradients, this lane's components
+		MatV m = mat_of<MM>(b, ph, i);
+#pragma unroll
+		for (int k = 0; k < 3; k++) {
+			if (nj[k] >= 0) {
+				double v[2];
+				ld2(nb[2 * a.cslot[k * n + i] + gp], min(nj[k], hd.y - 1), v);  // an own cell's neighbours are staged
+				o[0] += v[0];
+				o[1] += v[1];
+			} else {
+				ghost_gradient_adj(b, a, -1 - nj[k], own && gp == 0, pi, m, nbb[k], pb);
+			}
+		}
+		adj_finish<MODE>(a, i, gp, own, pi, m, o, pb, wa, wb);
+	}
+}
+
 // boundary-parameter adjoints: one workgroup per boundary object sums the
 // per-edge entries of that object's run of edges, in an order fixed by the
 // launch shape (strided partial sums, then a tree over the workgroup)
@@ -1531,8 +1706,9 @@ void carve_work(AdjWork& W, Carve& cv, int nck, size_t nrec, size_t nc, size_t n
 	W.a.Wn = cv.take<double>(n4);
 	W.a.Ws = cv.take<double>(n4);
 	W.a.Acc = cv.take<double>(n4);
-	W.a.Pb = cv.take<double>(n4);
-	W.a.Gb = cv.take<double>(n8);
+	bool tile = edge_buffer && !geo;
+	W.a.Pb = tile ? nullptr : cv.take<double>(n4);
+	W.a.Gb = tile ? nullptr : cv.take<double>(n8);
 	W.a.Ea = edge_buffer ? cv.take<double>((size_t)EA * ne) : nullptr;
 	W.a.Ebc = cv.take<double>(8 * ne);
 	W.a.bcbar = cv.take<double>(4 * (size_t)(nbc > 0 ? nbc : 1));
@@ -1657,30 +1833,43 @@ void launch_adj_grad(cfd2d_ctx* c, AdjWork* A, double wa, double wb, int mode)
 	else hipLaunchKernelGGL((k_adj_grad<MM, LSQ, 2, GEO>), g, blk, 0, c->st, c->b, c->ph, A->a, wa, wb);
 }
 
-// GEO: geometry adjoints too (the length and area terms take the stage's
-// fluxes from the edge reverse's own flux evaluation)
+template <bool MM, bool LSQ>
+void launch_adj_tile(cfd2d_ctx* c, AdjWork* A, double wa, double wb, int mode)
+{
+	dim3 g(c->b.ntiles), blk((2 * c->b.tsc + 63) / 64 * 64);
+	if (mode == 0) hipLaunchKernelGGL((k_adj_tile<MM, LSQ, 0>), g, blk, 0, c->st, c->b, c->ph, A->a, wa, wb);
+	else if (mode == 1) hipLaunchKernelGGL((k_adj_tile<MM, LSQ, 1>), g, blk, 0, c->st, c->b, c->ph, A->a, wa, wb);
+	else hipLaunchKernelGGL((k_adj_tile<MM, LSQ, 2>), g, blk, 0, c->st, c->b, c->ph, A->a, wa, wb);
+}
+
+// One stage's reverse.  GEO: geometry adjoints too (the length and area terms
+// take the stage's fluxes from the edge reverse's own flux evaluation)
 template <bool MM, bool GEO>
 void launch_adj_stage(cfd2d_ctx* c, AdjWork* A, double wa, double wb, int mode)
 {
+	bool lsq = c->p.gradient == CFD2D_GRAD_LSQ;
+	dim3 ge(grid_of(2 * c->ne)), blk(BLOCK);
 	if (c->p.flux == CFD2D_FLUX_HLLC || c->p.flux == CFD2D_FLUX_GODUNOV) {
 		// VJPs heavy in VALU work: once per edge, through the edge buffer
 		if (c->p.flux == CFD2D_FLUX_HLLC)
-			hipLaunchKernelGGL((k_adj_edge<MM, CFD2D_FLUX_HLLC, GEO>), dim3(grid_of(2 * c->ne)), dim3(BLOCK), 0,
-			                   c->st, c->b, c->ph, A->a, wb);
+			hipLaunchKernelGGL((k_adj_edge<MM, CFD2D_FLUX_HLLC, GEO>), ge, blk, 0, c->st, c->b, c->ph, A->a, wb);
 		else
-			hipLaunchKernelGGL((k_adj_edge<MM, CFD2D_FLUX_GODUNOV, GEO>), dim3(grid_of(2 * c->ne)), dim3(BLOCK), 0,
-			                   c->st, c->b, c->ph, A->a, wb);
-		hipLaunchKernelGGL(k_adj_cell, dim3(grid_of(c->nc)), dim3(BLOCK), 0, c->st, c->b, A->a);
+			hipLaunchKernelGGL((k_adj_edge<MM, CFD2D_FLUX_GODUNOV, GEO>), ge, blk, 0, c->st, c->b, c->ph, A->a, wb);
+		if (!GEO) {
+			if (lsq) launch_adj_tile<MM, true>(c, A, wa, wb, mode);
+			else launch_adj_tile<MM, false>(c, A, wa, wb, mode);
+			return;
+		}
+		hipLaunchKernelGGL(k_adj_cell, dim3(grid_of(2 * c->nc)), blk, 0, c->st, c->b, A->a);
 	} else {
 		// cheap VJP: evaluated from both sides, no edge buffer; the geometry
 		// terms (both sides' adjoints per edge) and the stage's fluxes by edge
-		hipLaunchKernelGGL((k_adj_face<MM, CFD2D_FLUX_LAX>), dim3(grid_of(2 * c->nc)), dim3(BLOCK), 0, c->st,
-		                   c->b, c->ph, A->a, wb);
+		hipLaunchKernelGGL((k_adj_face<MM, CFD2D_FLUX_LAX>), dim3(grid_of(2 * c->nc)), blk, 0, c->st, c->b, c->ph,
+		                   A->a, wb);
 		if (GEO)
-			hipLaunchKernelGGL((k_adj_edge<MM, CFD2D_FLUX_LAX, true, true>), dim3(grid_of(2 * c->ne)), dim3(BLOCK), 0,
-			                   c->st, c->b, c->ph, A->a, wb);
+			hipLaunchKernelGGL((k_adj_edge<MM, CFD2D_FLUX_LAX, true, true>), ge, blk, 0, c->st, c->b, c->ph, A->a, wb);
 	}
-	if (c->p.gradient == CFD2D_GRAD_LSQ) launch_adj_grad<MM, true, GEO>(c, A, wa, wb, mode);
+	if (lsq) launch_adj_grad<MM, true, GEO>(c, A, wa, wb, mode);
 	else launch_adj_grad<MM, false, GEO>(c, A, wa, wb, mode);
 }
 

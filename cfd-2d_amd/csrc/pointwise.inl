@@ -196,7 +196,7 @@ __global__ __launch_bounds__(BLOCK) void k_pw_vjp(int kind, int n, const double*
 	double fb[4], Lb[4], Rb[4], nb[2];
 	for (int q = 0; q < 4; q++) fb[q] = fbar[4 * (size_t)i + q];
 	if (kind == CFD2D_FLUX_LAX) lax_vjp(L, R, r[8], r[9], K.GAM, 1.0 / (K.GAM - 1.0), fb, Lb, Rb, nb);
-	else if (kind == CFD2D_FLUX_HLLC) hllc_vjp(L, R, r[8], r[9], K.GAM, fb, Lb, Rb, nb);
+	else if (kind == CFD2D_FLUX_HLLC) hllc_vjp(L, R, r[8], r[9], K.GAM, K.IAGAM, fb, Lb, Rb, nb);
 	else godunov_vjp(L, R, r[8], r[9], K, max_newton, fb, Lb, Rb, nb);
 	double* o = out + 10 * (size_t)i;
 	for (int q = 0; q < 4; q++) {
